@@ -256,9 +256,297 @@ __device__ float march2d_group(const TS *__restrict__ img, int W, int H, float o
   return pix;
 }
 
-// One lane per (detector pixel, view, batch item).
+// =====================================================================================
+// Forward through a pair copy of the image.  Element (x, y) of the copy holds the column
+// pair [v(x, y), v(x, y + 1)], x in [-2, W + 1], y in [-2, H], x fastest, zeros outside
+// the image; the elements of x and x + 1 together are the four neighbours of cell (x, y),
+// so a sample is ONE load at element alignment (16 bytes f32, 8 bytes 16-bit types) and
+// needs no bounds test: the coordinate is clamped into [-2, W] x [-2, H], where the cells
+// outside [-1, W) hold zeros only, exactly what the reference's border gives.
+//
+// What bound the direct march (march2d above): about 100 VALU instructions per sample (the
+// neighbours' bounds tests, 64-bit addresses and selects of the shared-ray version, the
+// iteration cap) around loads whose latency nothing covered.  Here a sample takes 39, and a
+// wave's load 22 cycles of the texture-address unit (16 for one 128-byte line per quad):
+// that unit is 88% busy and VALU issue at 0.39 of its 0.44-0.5 per SIMD and cycle.  Parallel
+// 256^2 / 180 views x 363 / step 0.2: 32 images 4300 -> 1420 us, one 282 -> 94; fan 512^2 /
+// 360 x 725 / step 0.5: 535 -> 158; fan 301 x 277 f16, spacing 0.7, one image: 522 -> 124.
+// A second copy with x and y exchanged, for rays along y, was no faster (1496 us, 180 us):
+// a quad's four samples span less than two pixels at these steps.
+// =====================================================================================
+template <typename TS> struct PairLoad {
+  typedef uint32_t raw __attribute__((ext_vector_type(2), aligned(4)));
+  static constexpr int kShift = 2;  // bytes of an element, log2
+};
+template <> struct PairLoad<float> {
+  typedef float raw __attribute__((ext_vector_type(4), aligned(8)));
+  static constexpr int kShift = 3;
+};
+
+__host__ __device__ inline int pair_cols(int W) { return W + 4; }
+__host__ __device__ inline int pair_rows(int H) { return H + 3; }
+
+// One lane per element.
+template <typename TS>
+__global__ void __launch_bounds__(256)
+build_pairs_kernel(const TS *__restrict__ img, TS *__restrict__ pairs, int H, int W) {
+  const int cx = blockIdx.x * 256 + threadIdx.x, cy = blockIdx.y;
+  const int Wp = pair_cols(W);
+  if (cx >= Wp) return;
+  const TS *im = img + (size_t)blockIdx.z * H * W;
+  const int x = cx - 2, y = cy - 2;
+  const bool vx = x >= 0 && x < W;
+  TS e[2];
+  e[0] = (vx && y >= 0 && y < H) ? im[(size_t)y * W + x] : zero_of<TS>();
+  e[1] = (vx && y + 1 >= 0 && y + 1 < H) ? im[(size_t)(y + 1) * W + x] : zero_of<TS>();
+  TS *o = pairs + (((size_t)blockIdx.z * pair_rows(H) + cy) * Wp + cx) * 2;
+  if constexpr (sizeof(TS) == 4) {
+    *reinterpret_cast<float2 *>(o) = make_float2(e[0], e[1]);
+  } else {
+    uint32_t w;
+    __builtin_memcpy(&w, e, 4);
+    *reinterpret_cast<uint32_t *>(o) = w;
+  }
+}
+
+// The image as the march sees it.  base is the pair copy moved by kPairBias bytes (see
+// pair_offset); fWp the copy's row length; c0 the float bias of the element index.
+struct PairImage {
+  const char *base;
+  float fWp, c0, fW, fH;
+};
+
+// Byte offset of cell (fx, fy) from PairImage::base.  fx + c0 and fy fWp + (fx + c0) are
+// exact integer-valued floats in [2^23, 2^24) (the host keeps the copy below 2^23
+// elements), so the bit pattern of the latter is 0x4B000000 + element index, and the shift
+// makes it 2^shift index + (0x4B000000 << shift) mod 2^32, which the base subtracts.
+template <typename TS>
+__device__ __forceinline__ uint32_t pair_offset(const PairImage &im, float fx, float fy) {
+  return __float_as_uint(fmaf(fy, im.fWp, fx + im.c0)) << PairLoad<TS>::kShift;
+}
+template <typename TS>
+__device__ __forceinline__ PairImage pair_image(const TS *pairs, int H, int W) {
+  constexpr uint32_t bias = 0x4B000000u << PairLoad<TS>::kShift;
+  const int Wp = pair_cols(W);
+  return {reinterpret_cast<const char *>(pairs) - (size_t)bias, (float)Wp, 0x1p23f + (float)(2 * Wp + 2), (float)W,
+          (float)H};
+}
+
+// x / s for the sampler, s the same for a whole image.
+//  kDivPow2: s a power of two, the exact product (pow2_reciprocal);
+//  kDivRefine: q = x RN(1/s), then twice q + (x - q s) RN(1/s).  The first correction leaves
+//    less than one ulp of error; from such a q, whose residual one FMA forms exactly, and a
+//    correctly rounded reciprocal the second gives the correctly rounded quotient
+//    (Markstein 1990), for s in [2^-60, 2^60].  Where a residual may be inexact or a product
+//    overflow (|x| < 2^-101, |x| > 2^67, infinities) the quotient may differ from x / s, but
+//    its sample does not: such a tiny quotient vanishes in (q + 0.5) - 0.5, and infinite,
+//    huge or NaN coordinates all sample zeros;
+//  kDivIeee: the division, for any s.
+enum { kDivPow2 = 1, kDivRefine = 2, kDivIeee = 0 };
+template <int DIV>
+__device__ __forceinline__ float div_spacing(float x, float s, float inv) {
+  if (DIV == kDivPow2) return x * inv;
+  if (DIV == kDivIeee) return x / s;
+  float q = x * inv;
+  q = fmaf(fmaf(-q, s, x), inv, q);
+  return fmaf(fmaf(-q, s, x), inv, q);
+}
+
+struct Ray2d {
+  float ox, oy, sx, sy, ix, iy, s0, s1, r0, r1;
+};
+
+// Cell and fractions of the sample at alpha a, and its load.
+template <typename TS, int DIV>
+__device__ __forceinline__ typename PairLoad<TS>::raw fetch2d(const PairImage &im, const Ray2d &r, float a,
+                                                              float &xd, float &yd) {
+  const float cx = div_spacing<DIV>(fmaf(a, r.r0, r.s0) - r.ox, r.sx, r.ix) + 0.5f;
+  const float cy = div_spacing<DIV>(fmaf(a, r.r1, r.s1) - r.oy, r.sy, r.iy) + 0.5f;
+  const float bx = __builtin_amdgcn_fmed3f(cx - 0.5f, -2.0f, im.fW);
+  const float by = __builtin_amdgcn_fmed3f(cy - 0.5f, -2.0f, im.fH);
+  const float fx = floorf(bx), fy = floorf(by);
+  xd = bx - fx;
+  yd = by - fy;
+  return *reinterpret_cast<const typename PairLoad<TS>::raw *>(im.base + pair_offset<TS>(im, fx, fy));
+}
+
+__device__ __forceinline__ float blend_pairs(float, PairLoad<float>::raw v, float xd, float yd) {
+  return lerp_ref(lerp_ref(v.x, v.z, xd), lerp_ref(v.y, v.w, xd), yd);
+}
+template <typename TS>
+__device__ __forceinline__ float blend_pairs(TS, typename PairLoad<TS>::raw v, float xd, float yd) {
+  TS a[2], b[2];
+  const uint32_t w0 = v.x, w1 = v.y;
+  __builtin_memcpy(a, &w0, 4);
+  __builtin_memcpy(b, &w1, 4);
+  return lerp_ref(lerp_ref(to_f32(a[0]), to_f32(b[0]), xd), lerp_ref(to_f32(a[1]), to_f32(b[1]), xd), yd);
+}
+
+// Value of lane J of this lane's group of G (all lanes of the group active): DPP quad_perm
+// for quads, row_newbcast for rows of 16.
+template <int G, int J>
+__device__ __forceinline__ float group_bcast(float f) {
+  static_assert(G == 4 || G == 16, "a quad or a row of lanes");
+  constexpr int ctrl = G == 4 ? J * 0x55 : 0x150 + J;
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), ctrl, 0xf, 0xf, true));
+}
+template <int G, int J = 0>
+__device__ __forceinline__ float group_sum(float pix, float f) {  // pix + f(0) + f(1) + ... in lane order
+  if constexpr (J < G) return group_sum<G, J + 1>(pix + group_bcast<G, J>(f), f);
+  return pix;
+}
+template <int G, int J = 0>
+__device__ __forceinline__ float group_max(float m, float f) {
+  if constexpr (J < G) return group_max<G, J + 1>(fmaxf(m, group_bcast<G, J>(f)), f);
+  return m;
+}
+
+// Emits nothing; the compiler moves no load across it (it would sink the load of the next
+// round below the loop's exit test, next to its use).
+__device__ __forceinline__ void keep_load_here() { asm volatile("" ::: "memory"); }
+
+// The march of march2d with the samples of one ray spread over G lanes: lane q of the group
+// takes samples q, q + G, ...  Each lane steps its own alpha by G float additions of step,
+// which are the additions of the one-lane recurrence, and every lane adds the G values of a
+// round in sample order, so all G lanes hold the one-lane sum, bit for bit; a lane past the
+// end adds -0.0, which changes no float.  The load of the next round is issued before the
+// current one is blended; positions past the end are clamped into the copy like any other.
+// The entrance sample and the tail are computed by all lanes alike.  CAP: with the reference
+// march's iteration cap (see proj2d_pairs_kernel).
+template <typename TS, int DIV, bool CAP, int G>
+__device__ __forceinline__ float march2d_pairs(const PairImage &im, const Ray2d &r, float amin, float amax,
+                                               float step, int q) {
+  typedef typename PairLoad<TS>::raw raw;
+  if (!(amin < amax)) return 0.0f;
+  const int cap = CAP ? march_cap(amin, amax, step) : 0;
+  float xa, ya, xb, yb;
+  raw va = fetch2d<TS, DIV>(im, r, amin, xa, ya), vb;
+  float pix = fmaf(0.5f, blend_pairs(TS{}, va, xa, ya), 0.0f);
+  float last = amin;  // alpha of this lane's last sample so far
+  float a = amin + step;
+#pragma unroll
+  for (int j = 1; j < G; ++j) {
+    const float nx = a + step;
+    a = q >= j ? nx : a;
+  }
+  int it = 0;
+  va = fetch2d<TS, DIV>(im, r, a, xa, ya);
+  // Two rounds per pass, so that no cell moves between registers.  The first lane's alpha
+  // decides for the group: alpha only grows, so the samples that exist are a prefix of a round.
+  while (group_bcast<G, 0>(a) < amax && (!CAP || it < cap)) {
+    float an = a;
+#pragma unroll
+    for (int j = 0; j < G; ++j) an += step;
+    vb = fetch2d<TS, DIV>(im, r, an, xb, yb);
+    const bool oka = a < amax && (!CAP || it + q < cap);
+    last = oka ? a : last;
+    pix = group_sum<G>(pix, oka ? blend_pairs(TS{}, va, xa, ya) : -0.0f);
+    a = an;
+#pragma unroll
+    for (int j = 0; j < G; ++j) a += step;
+    va = fetch2d<TS, DIV>(im, r, a, xa, ya);
+    const bool okb = an < amax && (!CAP || it + G + q < cap);
+    last = okb ? an : last;
+    pix = group_sum<G>(pix, okb ? blend_pairs(TS{}, vb, xb, yb) : -0.0f);
+    it += 2 * G;
+    keep_load_here();
+  }
+  pix *= step;
+  if (pix > 0.0f) {
+    const float alast = group_max<G>(last, last);
+    va = fetch2d<TS, DIV>(im, r, alast, xa, ya);
+    vb = fetch2d<TS, DIV>(im, r, amax, xb, yb);
+    const float flast = blend_pairs(TS{}, va, xa, ya);
+    pix = fmaf(-(0.5f * step), flast, pix);
+    const float rest = amax - ((alast + step) - step);
+    pix = fmaf(0.5f * rest, flast, pix);
+    pix = fmaf(0.5f * rest, blend_pairs(TS{}, vb, xb, yb), pix);
+  }
+  return pix;
+}
+
+// Source and direction of the ray of detector pixel d in one view.
 // Parallel: project_2Dpar_beam_kernel, par_projector_2D_CudaKernel.cu.cc:104-147.
 // Fan:      project_2Dfan_beam_kernel, fan_projector_2D_CudaKernel.cu.cc:104-149.
+template <bool FAN>
+__device__ __forceinline__ void ray2d(const float *__restrict__ ray, const float *__restrict__ vorigin, float dorigin,
+                                      const float *__restrict__ vspacing, float dspacing,
+                                      const float *__restrict__ sid_p, const float *__restrict__ sdd_p, int H, int W,
+                                      int d, float &ox, float &oy, float &sx, float &sy, float &s0, float &s1,
+                                      float &r0, float &r1) {
+  sx = vspacing[1];
+  sy = vspacing[0];
+  ox = vorigin[1];
+  oy = vorigin[0];
+  const float c0 = ray[0], c1 = ray[1];
+  const float u0 = -c1, u1 = c0;
+  const float u = i2p((float)d, dorigin, dspacing);
+  if (!FAN) {
+    const float a = (((float)W * sx) * (float)W) * sx;
+    const float sid = sqrtf(fmaf(((float)H * sy) * (float)H, sy, a)) * 1.2f;
+    s0 = fmaf(u0, u, c0 * (-sid));
+    s1 = fmaf(u1, u, c1 * (-sid));
+    r0 = c0;
+    r1 = c1;
+  } else {
+    const float sid = *sid_p, sdd = *sdd_p;
+    s0 = c0 * (-sid);
+    s1 = c1 * (-sid);
+    const float dx = fmaf(u0, u, fmaf(c0, sdd, s0));
+    const float dy = fmaf(u1, u, fmaf(c1, sdd, s1));
+    const float ex = dx - s0, ey = dy - s1;
+    const float nrm = 1.0f / sqrtf(fmaf(ey, ey, ex * ex));
+    r0 = ex * nrm;
+    r1 = ey * nrm;
+  }
+}
+
+// One projection reading the pair copy: G lanes per (detector pixel, view), batch items in
+// blockIdx.z.  A ray needs no iteration cap when step >= 2^-20 |alpha| over its interval
+// (at least 8 ulp of alpha, so each addition advances by at least 15/16 step and the march
+// ends before the cap of 1.25 (amax - amin) / step + 16); the choice is uniform per wave and
+// never changes a result.
+template <typename TS, bool FAN, int G>
+__global__ void __launch_bounds__(64)
+proj2d_pairs_kernel(const TS *__restrict__ pairs, float *__restrict__ sino, const float *__restrict__ rays,
+                    const float *__restrict__ vorigin, const float *__restrict__ dorigin,
+                    const float *__restrict__ vspacing, const float *__restrict__ dspacing,
+                    const float *__restrict__ sid_p, const float *__restrict__ sdd_p, int H, int W, int n, int det,
+                    float step_factor) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int d = t / G, q = t % G;
+  const int view = blockIdx.y, b = blockIdx.z;
+  if (d >= det) return;  // the G lanes of a pixel share d
+  const size_t vb = (size_t)b * n + view;
+  Ray2d r;
+  ray2d<FAN>(rays + vb * 2, vorigin + b * 2, dorigin[b], vspacing + b * 2, dspacing[b], sid_p + b, sdd_p + b, H, W, d,
+             r.ox, r.oy, r.sx, r.sy, r.s0, r.s1, r.r0, r.r1);
+  const float step = step_factor * fminf(r.sx, r.sy);
+  float amin, amax;
+  clip2d(W, H, r.ox, r.oy, r.sx, r.sy, r.s0, r.s1, r.r0, r.r1, amin, amax);
+  const PairImage im = pair_image(pairs + (size_t)b * pair_rows(H) * pair_cols(W) * 2, H, W);
+  r.ix = pow2_reciprocal(r.sx);
+  r.iy = pow2_reciprocal(r.sy);
+  const bool pow2 = r.ix != 0.0f && r.iy != 0.0f;  // spacings are per batch item: uniform over the block
+  const bool mid = fminf(r.sx, r.sy) >= 0x1p-60f && fmaxf(r.sx, r.sy) <= 0x1p60f;
+  const bool plain = !(fmaxf(fabsf(amin), fabsf(amax)) * 0x1p-20f > step);
+  float pix;
+  if (!(step > 0.0f)) {
+    pix = __builtin_nanf("");
+  } else if (!__all(plain) || !(pow2 || mid)) {
+    pix = march2d_pairs<TS, kDivIeee, true, G>(im, r, amin, amax, step, q);
+  } else if (pow2) {
+    pix = march2d_pairs<TS, kDivPow2, false, G>(im, r, amin, amax, step, q);
+  } else {
+    r.ix = 1.0f / r.sx;
+    r.iy = 1.0f / r.sy;
+    pix = march2d_pairs<TS, kDivRefine, false, G>(im, r, amin, amax, step, q);
+  }
+  const float a = r.r0 * r.sx, c = r.r1 * r.sy;
+  if (q == 0) sino[vb * det + d] = pix * sqrtf(fmaf(c, c, a * a));
+}
+
+// One lane per (detector pixel, view, batch item), reading the image itself.
 // G lanes per pixel (1, or 4 with march2d_group for launches with few rays).
 template <typename TS, bool FAN, int G>
 __global__ void __launch_bounds__(256)
@@ -271,31 +559,10 @@ proj2d_kernel(const TS *__restrict__ vol, float *__restrict__ sino, const float 
   const int d = t / G, q = t % G;
   const int view = blockIdx.y, b = blockIdx.z;
   if (d >= det) return;  // the G lanes of a pixel share d
-  const float sx = vspacing[b * 2 + 1], sy = vspacing[b * 2 + 0];
-  const float ox = vorigin[b * 2 + 1], oy = vorigin[b * 2 + 0];
   const size_t vb = (size_t)b * n + view;
-  const float c0 = rays[vb * 2 + 0], c1 = rays[vb * 2 + 1];
-  const float u0 = -c1, u1 = c0;
-  const float u = i2p((float)d, dorigin[b], dspacing[b]);
-  float s0, s1, r0, r1;
-  if (!FAN) {
-    const float a = (((float)W * sx) * (float)W) * sx;
-    const float sid = sqrtf(fmaf(((float)H * sy) * (float)H, sy, a)) * 1.2f;
-    s0 = fmaf(u0, u, c0 * (-sid));
-    s1 = fmaf(u1, u, c1 * (-sid));
-    r0 = c0;
-    r1 = c1;
-  } else {
-    const float sid = sid_p[b], sdd = sdd_p[b];
-    s0 = c0 * (-sid);
-    s1 = c1 * (-sid);
-    const float dx = fmaf(u0, u, fmaf(c0, sdd, s0));
-    const float dy = fmaf(u1, u, fmaf(c1, sdd, s1));
-    const float ex = dx - s0, ey = dy - s1;
-    const float nrm = 1.0f / sqrtf(fmaf(ey, ey, ex * ex));
-    r0 = ex * nrm;
-    r1 = ey * nrm;
-  }
+  float sx, sy, ox, oy, s0, s1, r0, r1;
+  ray2d<FAN>(rays + vb * 2, vorigin + b * 2, dorigin[b], vspacing + b * 2, dspacing[b], sid_p + b, sdd_p + b, H, W, d,
+             ox, oy, sx, sy, s0, s1, r0, r1);
   const float step = step_factor * fminf(sx, sy);
   const TS *img = vol + (size_t)b * H * W;
   // spacings are per batch item, so the choice is uniform over the block
@@ -416,11 +683,37 @@ static void launch_proj2d_g(dim3 grid, const void *volume, int dtype, int H, int
         (const _Float16 *)volume, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det, step_factor);
 }
 
+// Rays per launch below which a ray gets 16 lanes instead of 4: with 4 the launch would have
+// less than two waves per SIMD, each waiting for its own latencies (64^2 / 60 views x 95, 5700
+// rays: 11 against 18 us; 16650 rays: 25 against 31; 65340 rays: 119 against 94 the other way,
+// the 16 broadcasts of a round costing more than the latency they hide).
+constexpr long long kRowRayLimit = 32768;
+
+template <typename TS, bool FAN>
+static void launch_pairs(const void *volume, int batch, int H, int W, const float *vo, const float *dor,
+                         const float *vs, const float *ds, const float *sid, const float *sdd, const float *rays, int n,
+                         int det, float step_factor, float *sino, void *ws, hipStream_t s) {
+  TS *pairs = (TS *)ws;
+  build_pairs_kernel<TS><<<dim3((unsigned)((pair_cols(W) + 255) / 256), (unsigned)pair_rows(H), (unsigned)batch),
+                           dim3(256), 0, s>>>((const TS *)volume, pairs, H, W);
+  const int G = (long long)det * n * batch < kRowRayLimit ? 16 : 4;
+  // one wave per block: the rays of a view differ in length, and the dispatch evens out
+  // single waves best (256-lane blocks: 2168 against 1922 us for 16 fan 512^2 images, 171
+  // against 158 us for one; a batch of 32 parallel 256^2 images is the same)
+  const dim3 grid((unsigned)(((long long)G * det + 63) / 64), n, batch);
+  if (G == 16)
+    proj2d_pairs_kernel<TS, FAN, 16><<<grid, dim3(64), 0, s>>>(pairs, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n,
+                                                               det, step_factor);
+  else
+    proj2d_pairs_kernel<TS, FAN, 4><<<grid, dim3(64), 0, s>>>(pairs, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n,
+                                                              det, step_factor);
+}
+
 template <bool FAN>
 static int launch_proj2d(const char *name, const void *volume, int dtype, int batch, int H, int W,
                          const float *vo, const float *dor, const float *vs, const float *ds,
                          const float *sid, const float *sdd, const float *rays_p, int n, int det,
-                         float step_factor, float *sino, hipStream_t s) {
+                         float step_factor, float *sino, void *ws, size_t ws_bytes, bool use_ws, hipStream_t s) {
   clear_error();
   PYRONN_CHECK_ARG(volume && vo && dor && vs && ds && rays_p && sino, "%s: null pointer", name);
   PYRONN_CHECK_ARG(!FAN || (sid && sdd), "%s: null source distances", name);
@@ -430,6 +723,25 @@ static int launch_proj2d(const char *name, const void *volume, int dtype, int ba
   PYRONN_CHECK_ARG((long long)H * W < INT32_MAX, "%s: image too large", name);
   PYRONN_CHECK_ARG(step_factor > 0.0f, "%s: step factor must be > 0", name);
   PYRONN_CHECK_ARG(det <= INT32_MAX / 4, "%s: too many detector pixels", name);
+  if (use_ws) {
+    const size_t need = pyronn_projection2d_workspace_size(batch, H, W, dtype);
+    PYRONN_CHECK_ARG(need > 0, "%s: no pair copy for a %dx%d image", name, H, W);
+    PYRONN_CHECK_ARG(ws != nullptr, "%s: null workspace", name);
+    PYRONN_CHECK_ARG(((uintptr_t)ws & 15) == 0, "%s: workspace must be 16-byte aligned", name);
+    if (ws_bytes < need) {
+      set_error("%s: workspace %zu bytes < required %zu", name, ws_bytes, need);
+      return PYRONN_ERR_WORKSPACE;
+    }
+    if (dtype == PYRONN_F32)
+      launch_pairs<float, FAN>(volume, batch, H, W, vo, dor, vs, ds, sid, sdd, rays_p, n, det, step_factor, sino, ws, s);
+    else if (dtype == PYRONN_BF16)
+      launch_pairs<bf16s, FAN>(volume, batch, H, W, vo, dor, vs, ds, sid, sdd, rays_p, n, det, step_factor, sino, ws, s);
+    else
+      launch_pairs<_Float16, FAN>(volume, batch, H, W, vo, dor, vs, ds, sid, sdd, rays_p, n, det, step_factor, sino, ws,
+                                  s);
+    PYRONN_CHECK_LAUNCH(name);
+    return PYRONN_OK;
+  }
   // Few rays (one lane each would leave most SIMDs with a handful of latency-bound waves):
   // four lanes per ray.  Both variants give the same bits.
   const long long nrays = (long long)det * n * batch;
@@ -484,7 +796,7 @@ extern "C" int pyronn_parallel_projection2d(const void *volume, int volume_dtype
                                             pyronn_stream_t stream) {
   return launch_proj2d<false>("parallel_projection2d", volume, volume_dtype, batch, H, W,
                               volume_origin, detector_origin, volume_spacing, detector_spacing,
-                              nullptr, nullptr, ray_vectors, n_views, det, step_factor, sinogram,
+                              nullptr, nullptr, ray_vectors, n_views, det, step_factor, sinogram, nullptr, 0, false,
                               (hipStream_t)stream);
 }
 
@@ -500,8 +812,41 @@ extern "C" int pyronn_fan_projection2d(const void *volume, int volume_dtype, int
   return launch_proj2d<true>("fan_projection2d", volume, volume_dtype, batch, H, W, volume_origin,
                              detector_origin, volume_spacing, detector_spacing,
                              source_2_isocenter_distance, source_2_detector_distance,
-                             central_ray_vectors, n_views, det, step_factor, sinogram,
+                             central_ray_vectors, n_views, det, step_factor, sinogram, nullptr, 0, false,
                              (hipStream_t)stream);
+}
+
+extern "C" size_t pyronn_projection2d_workspace_size(int batch, int H, int W, int volume_dtype) {
+  if (batch <= 0 || H <= 0 || W <= 0 || !dtype_ok(volume_dtype)) return 0;
+  // the element index, biased by 2 Wp + 2 and 2^23, has to stay below 2^24 (pair_offset)
+  const long long elems = (long long)pair_cols(W) * pair_rows(H);
+  if (W > (1 << 23) || H > 65532 || elems >= (1 << 23)) return 0;
+  return align_up((size_t)batch * (size_t)elems * 2 * dtype_bytes(volume_dtype), 256);
+}
+
+extern "C" int pyronn_parallel_projection2d_ws(const void *volume, int volume_dtype, int batch, int H, int W,
+                                               const float *volume_origin, const float *detector_origin,
+                                               const float *volume_spacing, const float *detector_spacing,
+                                               const float *ray_vectors, int n_views, int det, float step_factor,
+                                               float *sinogram, void *workspace, size_t workspace_bytes,
+                                               pyronn_stream_t stream) {
+  return launch_proj2d<false>("parallel_projection2d_ws", volume, volume_dtype, batch, H, W, volume_origin,
+                              detector_origin, volume_spacing, detector_spacing, nullptr, nullptr, ray_vectors,
+                              n_views, det, step_factor, sinogram, workspace, workspace_bytes, true,
+                              (hipStream_t)stream);
+}
+
+extern "C" int pyronn_fan_projection2d_ws(const void *volume, int volume_dtype, int batch, int H, int W,
+                                          const float *volume_origin, const float *detector_origin,
+                                          const float *volume_spacing, const float *detector_spacing,
+                                          const float *source_2_isocenter_distance,
+                                          const float *source_2_detector_distance, const float *central_ray_vectors,
+                                          int n_views, int det, float step_factor, float *sinogram, void *workspace,
+                                          size_t workspace_bytes, pyronn_stream_t stream) {
+  return launch_proj2d<true>("fan_projection2d_ws", volume, volume_dtype, batch, H, W, volume_origin,
+                             detector_origin, volume_spacing, detector_spacing, source_2_isocenter_distance,
+                             source_2_detector_distance, central_ray_vectors, n_views, det, step_factor, sinogram,
+                             workspace, workspace_bytes, true, (hipStream_t)stream);
 }
 
 extern "C" int pyronn_parallel_backprojection2d(const void *sinogram, int sinogram_dtype,

@@ -174,19 +174,28 @@ at::Tensor proj2d(bool fan, const at::Tensor &volume, at::IntArrayRef projection
   const int dt = dtype_code(vol, op);
   at::Tensor out = at::empty({B, n, det}, vol.options().dtype(at::kFloat));
   if (empty_output(out)) return out;
+  // the pair copy of the images that the projection samples; none for images too large for it
+  const size_t ws = pyronn_projection2d_workspace_size((int)B, (int)H, (int)W, dt);
+  at::Tensor work;
+  if (ws) work = at::empty({(int64_t)ws}, vol.options().dtype(at::kByte));
+  const float *vop = g.vo.data_ptr<float>(), *dop = g.dor.data_ptr<float>(), *vsp = g.vs.data_ptr<float>(),
+              *dsp = g.ds.data_ptr<float>(), *rp = g.rays.data_ptr<float>();
+  const float *sidp = fan ? g.sid.data_ptr<float>() : nullptr, *sddp = fan ? g.sdd.data_ptr<float>() : nullptr;
+  float *outp = out.data_ptr<float>();
+  const pyronn_stream_t st = cur_stream(vol);
   int rc;
-  if (fan)
-    rc = pyronn_fan_projection2d(vol.data_ptr(), dt, (int)B, (int)H, (int)W, g.vo.data_ptr<float>(),
-                                 g.dor.data_ptr<float>(), g.vs.data_ptr<float>(), g.ds.data_ptr<float>(),
-                                 g.sid.data_ptr<float>(), g.sdd.data_ptr<float>(),
-                                 g.rays.data_ptr<float>(), (int)n, (int)det, (float)step_size,
-                                 out.data_ptr<float>(), cur_stream(vol));
+  if (ws && fan)
+    rc = pyronn_fan_projection2d_ws(vol.data_ptr(), dt, (int)B, (int)H, (int)W, vop, dop, vsp, dsp, sidp, sddp, rp,
+                                    (int)n, (int)det, (float)step_size, outp, work.data_ptr(), ws, st);
+  else if (ws)
+    rc = pyronn_parallel_projection2d_ws(vol.data_ptr(), dt, (int)B, (int)H, (int)W, vop, dop, vsp, dsp, rp, (int)n,
+                                         (int)det, (float)step_size, outp, work.data_ptr(), ws, st);
+  else if (fan)
+    rc = pyronn_fan_projection2d(vol.data_ptr(), dt, (int)B, (int)H, (int)W, vop, dop, vsp, dsp, sidp, sddp, rp,
+                                 (int)n, (int)det, (float)step_size, outp, st);
   else
-    rc = pyronn_parallel_projection2d(vol.data_ptr(), dt, (int)B, (int)H, (int)W,
-                                      g.vo.data_ptr<float>(), g.dor.data_ptr<float>(),
-                                      g.vs.data_ptr<float>(), g.ds.data_ptr<float>(),
-                                      g.rays.data_ptr<float>(), (int)n, (int)det, (float)step_size,
-                                      out.data_ptr<float>(), cur_stream(vol));
+    rc = pyronn_parallel_projection2d(vol.data_ptr(), dt, (int)B, (int)H, (int)W, vop, dop, vsp, dsp, rp, (int)n,
+                                      (int)det, (float)step_size, outp, st);
   check_rc(rc, op);
   return out;
 }

@@ -53,6 +53,11 @@ _SIGS = {
                                               _vp]),
     "pyronn_fan_projection2d": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f,
                                      _vp, _vp]),
+    "pyronn_projection2d_workspace_size": (_sz, [_i, _i, _i, _i]),
+    "pyronn_parallel_projection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp,
+                                             _vp, _sz, _vp]),
+    "pyronn_fan_projection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f,
+                                        _vp, _vp, _sz, _vp]),
     "pyronn_fan_backprojection2d": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,
                                          _vp, _vp]),
     "pyronn_cone_projection3d_batched_workspace_size": (_sz, [_vp, _i, _i]),

@@ -1,0 +1,78 @@
+"""The 2D projections through the pair copy of the images: the dispatch's edges (lanes per ray,
+remainders of the ray groups, spacings of each division, the largest copy) against the oracle."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as orc
+from pyronn_layers import geometry as geo
+from pyronn_layers import native as nat
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(fan, img, sp, n, det, ds, step, sid, storage=torch.float32, arc=2 * math.pi, off=(0.0, 0.0)):
+    import pyronn_layers as pl
+    H, W = img.shape[-2:]
+    org = (geo.centred_origin((H, W), sp) + np.asarray(off)).astype(np.float32)
+    sp = np.asarray(sp, np.float32)
+    rays = geo.parallel_ray_vectors(n, arc).astype(np.float32)
+    do = np.float32(-(det - 1) / 2 * ds)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    x = dev(img)[None].to(storage)
+    geom = [dev(org)[None], dev([[do]]), dev(sp)[None], dev([[ds]])]
+    if fan:
+        out = pl.fan_projection2d(x, [n, det], *geom, dev([[sid]]), dev([[1.4 * sid]]), dev(rays)[None], step)
+        ref = orc.fan_forward(x[0].float().cpu().numpy(), rays, det, org, sp, do, np.float32(ds),
+                              sid=np.float32(sid), sdd=np.float32(1.4 * sid), step_factor=step)[0]
+    else:
+        out = pl.parallel_projection2d(x, [n, det], *geom, dev(rays)[None], step)
+        ref = orc.parallel_forward(x[0].float().cpu().numpy(), rays, det, org, sp, do, np.float32(ds),
+                                   step_factor=step)[0]
+    return out[0].cpu().numpy(), ref
+
+
+@pytest.mark.parametrize("fan", [False, True])
+@pytest.mark.parametrize("storage", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H, W, sp, n, det", [
+    (1, 1, (1.0, 1.0), 5, 3),            # one pixel; 16 lanes per ray, a partly filled wave
+    (3, 70, (0.5, 0.5), 9, 65),          # power-of-two spacing below the box's 0.5 mm edge
+    (70, 3, (0.7, 1.3), 9, 66),          # refined division, two spacings
+    (33, 31, (0.3, 0.3), 7, 61),         # coordinates below -1: the copy's second border cell
+    (40, 44, (0.9, 1.0), 300, 110),      # 33000 rays: 4 lanes per ray, det no multiple of 16
+    (24, 24, (1e-19, 1e-19), 3, 17),     # a spacing the refined division does not serve
+])
+def test_pairs_match_the_oracle(fan, storage, H, W, sp, n, det):
+    img = np.random.default_rng(H * 100 + W).normal(size=(H, W)).astype(np.float32)
+    ext = max(H * sp[0], W * sp[1])
+    got, ref = _run(fan, img, sp, n, det, 1.3 * ext / det, 0.2 if sp[0] > 0.1 else 0.5, 1.5 * ext, storage)
+    assert np.array_equal(got, ref, equal_nan=True), int((got != ref).sum())
+
+
+@pytest.mark.parametrize("fan", [False, True])
+def test_pairs_far_box_and_capped_march(fan):
+    # alpha of about 3e6 spacings at a step of 0.2: the additions are rounded (the capped march)
+    img = np.random.default_rng(5).normal(size=(20, 18)).astype(np.float32)
+    got, ref = _run(fan, img, (1.0, 1.0), 5, 33, 1.0, 0.2, 60.0, arc=0.3, off=(4.0e6, 3.0e6))
+    assert np.array_equal(got, ref, equal_nan=True)
+    got, ref = _run(fan, img, (1.0, 1.0), 5, 33, 1.0, 1e-3, 3.0e5 if fan else 60.0)
+    assert np.array_equal(got, ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("H, W", [(2049, 4084), (2050, 4084)])
+def test_pairs_largest_copy_and_the_first_image_past_it(H, W):
+    size = nat.lib().pyronn_projection2d_workspace_size(1, H, W, nat.F32)
+    assert (size > 0) == ((W + 4) * (H + 3) < 2 ** 23)
+    img = np.random.default_rng(H).normal(size=(H, W)).astype(np.float32)
+    got, ref = _run(False, img, (1.0, 1.0), 3, 400, 12.0, 0.5, 0.0)
+    assert np.array_equal(got, ref)
+
+
+def test_pairs_infinite_and_nan_pixels_reach_the_same_rays():
+    img = np.random.default_rng(8).normal(size=(16, 18)).astype(np.float32)
+    img[0, 3], img[15, 0], img[7, 17] = np.inf, np.nan, -np.inf
+    for sp in ((0.25, 0.25), (1.0, 1.0), (0.3, 0.6)):
+        got, ref = _run(False, img, sp, 40, 41, 0.5, 0.2, 0.0)
+        assert np.array_equal(got, ref, equal_nan=True)
