@@ -38,21 +38,22 @@ int dtype_code(const at::Tensor &t, const char *op) {
   return -1;
 }
 
-// Geometry tensor as float32 [B, shape...] contiguous on `dev`.  Accepts the
-// per-item shape without the batch dimension (broadcast to every item).
-at::Tensor geom(const at::Tensor &t, int64_t B, std::vector<int64_t> shape, const char *op,
-                const char *name, const at::Device &dev) {
-  int64_t per = 1;
-  for (auto s : shape) per *= s;
+// Geometry tensor as contiguous float32 on `dev`, `per` values for each batch item (the kernels
+// take its data as it lies, so its shape does not matter).  Accepts one item's values without
+// the batch dimension (broadcast to every item).  A tensor that already is all that is used as
+// it is: no view, conversion or copy is made for it.
+at::Tensor geom(const at::Tensor &t, int64_t B, int64_t per, const char *op, const char *name,
+                const at::Device &dev) {
+  if (t.scalar_type() == at::kFloat && t.device() == dev && t.numel() == B * per && t.layout() == at::kStrided &&
+      t.is_contiguous())
+    return t;
   at::Tensor g = t.to(dev, at::kFloat).contiguous();
   if (g.numel() == per) {
     g = g.reshape({1, per}).expand({B, per}).contiguous();
   }
   TORCH_CHECK(g.numel() == B * per, op, ": ", name, " has ", g.numel(), " elements, expected ", B,
               " x ", per);
-  std::vector<int64_t> full{B};
-  full.insert(full.end(), shape.begin(), shape.end());
-  return g.reshape(full);
+  return g;
 }
 
 // An empty output (no batch items, no views, a zero-sized volume or detector) needs no
@@ -86,11 +87,11 @@ at::Tensor cone_projection3d(const at::Tensor &volume, at::IntArrayRef projectio
   const int64_t B = vol.size(0), D = vol.size(1), H = vol.size(2), W = vol.size(3);
   const int64_t n = projection_shape[0], Hd = projection_shape[1], Wd = projection_shape[2];
   const auto dev = vol.device();
-  const at::Tensor org = geom(volume_origin, B, {3}, op, "volume_origin", dev);
-  const at::Tensor sp = geom(volume_spacing, B, {3}, op, "volume_spacing", dev);
-  const at::Tensor P = geom(projection_matrices, B, {n, 3, 4}, op, "projection_matrices", dev);
-  const at::Tensor st = geom(step_size, B, {1}, op, "step_size", dev);
-  const at::Tensor mu = geom(projection_multiplier, B, {1}, op, "projection_multiplier", dev);
+  const at::Tensor org = geom(volume_origin, B, 3, op, "volume_origin", dev);
+  const at::Tensor sp = geom(volume_spacing, B, 3, op, "volume_spacing", dev);
+  const at::Tensor P = geom(projection_matrices, B, n * 12, op, "projection_matrices", dev);
+  const at::Tensor st = geom(step_size, B, 1, op, "step_size", dev);
+  const at::Tensor mu = geom(projection_multiplier, B, 1, op, "projection_multiplier", dev);
   const int dt = dtype_code(vol, op);
   at::Tensor out = at::empty({B, n, Hd, Wd}, vol.options().dtype(at::kFloat));
   if (empty_output(out)) return out;
@@ -118,11 +119,11 @@ at::Tensor cone_backprojection3d(const at::Tensor &sinogram, at::IntArrayRef vol
   const int64_t B = sino.size(0), n = sino.size(1), Hd = sino.size(2), Wd = sino.size(3);
   const int64_t D = volume_shape[0], H = volume_shape[1], W = volume_shape[2];
   const auto dev = sino.device();
-  const at::Tensor org = geom(volume_origin, B, {3}, op, "volume_origin", dev);
-  const at::Tensor sp = geom(volume_spacing, B, {3}, op, "volume_spacing", dev);
-  const at::Tensor P = geom(projection_matrices, B, {n, 3, 4}, op, "projection_matrices", dev);
-  const at::Tensor st = geom(step_size, B, {1}, op, "step_size", dev);
-  const at::Tensor mu = geom(projection_multiplier, B, {1}, op, "projection_multiplier", dev);
+  const at::Tensor org = geom(volume_origin, B, 3, op, "volume_origin", dev);
+  const at::Tensor sp = geom(volume_spacing, B, 3, op, "volume_spacing", dev);
+  const at::Tensor P = geom(projection_matrices, B, n * 12, op, "projection_matrices", dev);
+  const at::Tensor st = geom(step_size, B, 1, op, "step_size", dev);
+  const at::Tensor mu = geom(projection_multiplier, B, 1, op, "projection_multiplier", dev);
   const int dt = dtype_code(sino, op);
   at::Tensor out = at::empty({B, D, H, W}, sino.options().dtype(at::kFloat));
   if (empty_output(out)) return out;
@@ -149,13 +150,13 @@ Geo2D geo2d(int64_t B, int64_t n, const at::Tensor &vo, const at::Tensor &dor, c
             const at::Tensor &ds, const at::Tensor *sid, const at::Tensor *sdd,
             const at::Tensor &rays, const char *op, const at::Device &dev) {
   Geo2D g;
-  g.vo = geom(vo, B, {2}, op, "volume_origin", dev);
-  g.dor = geom(dor, B, {1}, op, "detector_origin", dev);
-  g.vs = geom(vs, B, {2}, op, "volume_spacing", dev);
-  g.ds = geom(ds, B, {1}, op, "detector_spacing", dev);
-  if (sid) g.sid = geom(*sid, B, {1}, op, "source_2_isocenter_distance", dev);
-  if (sdd) g.sdd = geom(*sdd, B, {1}, op, "source_2_detector_distance", dev);
-  g.rays = geom(rays, B, {n, 2}, op, "ray_vectors", dev);
+  g.vo = geom(vo, B, 2, op, "volume_origin", dev);
+  g.dor = geom(dor, B, 1, op, "detector_origin", dev);
+  g.vs = geom(vs, B, 2, op, "volume_spacing", dev);
+  g.ds = geom(ds, B, 1, op, "detector_spacing", dev);
+  if (sid) g.sid = geom(*sid, B, 1, op, "source_2_isocenter_distance", dev);
+  if (sdd) g.sdd = geom(*sdd, B, 1, op, "source_2_detector_distance", dev);
+  g.rays = geom(rays, B, n * 2, op, "ray_vectors", dev);
   return g;
 }
 
