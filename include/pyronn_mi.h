@@ -244,6 +244,27 @@ int pyronn_fan_backprojection2d(const void *sinogram, int sinogram_dtype, int ba
                                 const float *central_ray_vectors, int H, int W, float *volume,
                                 pyronn_stream_t stream);
 
+/*
+ * The two 2D backprojections through a copy of the projections with a zero border in the
+ * workspace: the same results as the calls above bit for bit, faster.
+ * pyronn_backprojection2d_workspace_size gives 0 for 2^22 detector pixels or more; use the
+ * calls above there.
+ */
+size_t pyronn_backprojection2d_workspace_size(int batch, int n_views, int det, int sinogram_dtype);
+int pyronn_parallel_backprojection2d_ws(const void *sinogram, int sinogram_dtype, int batch,
+                                        int n_views, int det, const float *volume_origin,
+                                        const float *detector_origin, const float *volume_spacing,
+                                        const float *detector_spacing, const float *ray_vectors,
+                                        int H, int W, float *volume, void *workspace,
+                                        size_t workspace_bytes, pyronn_stream_t stream);
+int pyronn_fan_backprojection2d_ws(const void *sinogram, int sinogram_dtype, int batch, int n_views,
+                                   int det, const float *volume_origin, const float *detector_origin,
+                                   const float *volume_spacing, const float *detector_spacing,
+                                   const float *source_2_isocenter_distance,
+                                   const float *source_2_detector_distance,
+                                   const float *central_ray_vectors, int H, int W, float *volume,
+                                   void *workspace, size_t workspace_bytes, pyronn_stream_t stream);
+
 /* --------------------------------------------------------------------------
  * Batched cone operators over problems of different shapes and geometries.
  * No single counterpart in the reference: ConeProjection3DOp::Compute

@@ -77,6 +77,23 @@ __device__ __forceinline__ float rcp_fast(float w) {
 }
 __device__ __forceinline__ float rcp_rn(float w) { return rcp_fast_ok(w) ? rcp_fast(w) : 1.0f / w; }
 
+// 1.0f / sqrtf(t), both correctly rounded as the reference's square root and division are,
+// for t in [2^-100, 2^100]: from the hardware estimate of 1/sqrt(t), one Goldschmidt step
+// for the root g and for h = 1/(2 g), a last correction of g by its exact residual
+// (Markstein), and rcp_fast.  13 instructions against 26 for the two IEEE sequences.  Bit
+// equality over every t of the range is checked on the device by the test suite.  (2 h as
+// the reciprocal's estimate saves an instruction, but is wrong where g's mantissa is all
+// ones: 200 of the range's 1.7e9 floats.)
+__device__ __forceinline__ bool rcp_sqrt_ok(float t) { return t >= 0x1p-100f && t <= 0x1p100f; }
+__device__ __forceinline__ float rcp_sqrt_fast(float t) {
+  const float y = __builtin_amdgcn_rsqf(t);
+  float g = t * y, h = 0.5f * y;
+  const float r = fmaf(-h, g, 0.5f);
+  g = fmaf(g, r, g);
+  h = fmaf(h, r, h);
+  return rcp_fast(fmaf(fmaf(-g, g, t), h, g));
+}
+
 // Iteration cap of every ray march (the reference has none and would spin
 // forever when the step is below the float resolution of alpha).  At most 2^25
 // iterations: with a step of at least half a voxel and alpha below 2^23 voxels, no

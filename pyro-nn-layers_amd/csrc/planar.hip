@@ -664,6 +664,191 @@ back2d_kernel(const TS *__restrict__ sino, float *__restrict__ vol, const float 
   }
 }
 
+// =====================================================================================
+// Backprojection through a copy of the projections with a zero border: row (batch, view)
+// holds s(-2) .. s(det + 1), zeros outside the detector, so a linear sample is one pair load
+// and no bounds test, the coordinate clamped into [-2, det].
+//
+// The fan kernel is bound by VALU issue.  back2d_kernel above forms about 130 instructions
+// per update: per-view terms of the line intersection that are the same for every pixel, two
+// IEEE divisions by one denominator, an IEEE square root and its reciprocal.  Here a block
+// forms the per-view terms once, in LDS (kBackViews views at a time; every lane reads them
+// back with two broadcast reads), both quotients share one correctly rounded reciprocal
+// (div_spacing's two corrections), and rcp_sqrt_fast serves the weight: about 68 per update.
+// The parallel kernel's 15 leave it to the address path, one pair load per update.  512^2 fan,
+// 360 views x 725: 221 -> 133 us (8 images 1233 -> 805); 256^2 parallel, 180 views x 363: 45 ->
+// 23.5 us (32 images 309 -> 181).
+// =====================================================================================
+__host__ __device__ inline int row_len(int det) { return det + 4; }
+
+template <typename TS>
+__global__ void __launch_bounds__(256)
+build_rows_kernel(const TS *__restrict__ sino, TS *__restrict__ rows, int det, long long nrows) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= row_len(det)) return;
+  const int u = c - 2;
+  const bool in = u >= 0 && u < det;
+  for (long long r = blockIdx.y; r < nrows; r += gridDim.y)
+    rows[(size_t)r * row_len(det) + c] = in ? sino[(size_t)r * det + u] : zero_of<TS>();
+}
+
+template <typename TS> struct PairOf16 { typedef uint32_t raw __attribute__((aligned(2))); };
+
+// Linear sample of a bordered row at detector index si (the sampler's + 0.5 - 0.5 included).
+// base is the row moved by the bias of the offset's float form, as in pair_offset.
+template <typename TS>
+__device__ __forceinline__ float sample_row(const char *__restrict__ base, float fdet, float si) {
+  const float b = __builtin_amdgcn_fmed3f((si + 0.5f) - 0.5f, -2.0f, fdet);
+  const float f = floorf(b);
+  const uint32_t at = __float_as_uint(f + (0x1p23f + 2.0f)) << (sizeof(TS) == 4 ? 2 : 1);
+  float p0, p1;
+  if constexpr (sizeof(TS) == 4) {
+    const f32x2_a4 v = *reinterpret_cast<const f32x2_a4 *>(base + at);
+    p0 = v.x;
+    p1 = v.y;
+  } else {
+    const uint32_t w = *reinterpret_cast<const typename PairOf16<TS>::raw *>(base + at);
+    TS e[2];
+    __builtin_memcpy(e, &w, 4);
+    p0 = to_f32(e[0]);
+    p1 = to_f32(e[1]);
+  }
+  return lerp_ref(p0, p1, b - f);
+}
+
+// The terms of one view that no pixel changes.  Fan: source (srx, sry); b, d, g of the
+// intersection with the detector line through the reference's two points; (d0, d1) the
+// detector axis.  Parallel: (c0, -c1).
+struct alignas(16) ViewTerms {
+  float srx, sry, b, d, g, d0, d1, unused;
+};
+constexpr int kBackViews = 128;
+
+// The fan pixel's detector coordinate in mm and distance weight.  FAST: see back2d_rows_kernel.
+template <bool FAST>
+__device__ __forceinline__ void fan_pixel(const ViewTerms &v, float pcx, float pcy, float &s, float &dw) {
+  const float a = pcx - v.srx, c = pcy - v.sry;
+  const float den = fmaf(-c, v.d, a * v.b);
+  const float e = fmaf(-pcy, v.srx, pcx * v.sry);
+  const float nx = fmaf(-a, v.g, e * v.d), ny = fmaf(-c, v.g, e * v.b);
+  float ix, iy;
+  if (FAST) {
+    const float r = rcp_fast(den);
+    ix = div_spacing<kDivRefine>(nx, den, r);
+    iy = div_spacing<kDivRefine>(ny, den, r);
+  } else {
+    ix = nx / den;
+    iy = ny / den;
+  }
+  s = fmaf(iy, v.d1, ix * v.d0);
+  if (den < 0.000001f && den > -0.000001f) s = __builtin_nanf("");  // helper_geometry_gpu.h:28-44
+  const float t = fmaf(c, c, a * a);
+  dw = (FAST && rcp_sqrt_ok(t)) ? rcp_sqrt_fast(t) : rcp_rn(sqrtf(t));
+}
+
+template <typename TS, bool FAN, bool FAST, int DIV, int P>
+__device__ __forceinline__ void back2d_rows(const TS *__restrict__ rows, const float *__restrict__ rb, int n, int det,
+                                            float pcx, const float *pcy, float do_, float ds, float ids, float sid,
+                                            float sdd, ViewTerms *terms, float *val) {
+  const float fdet = (float)det;
+  constexpr uint32_t bias = 0x4B000000u << (sizeof(TS) == 4 ? 2 : 1);
+  const char *base = reinterpret_cast<const char *>(rows) - (size_t)bias;
+  for (int v0 = 0; v0 < n; v0 += kBackViews) {
+    const int nv = n - v0 < kBackViews ? n - v0 : kBackViews;
+    __syncthreads();
+    for (int k = threadIdx.x; k < nv; k += blockDim.x) {
+      const float c0 = rb[(v0 + k) * 2 + 0], c1 = rb[(v0 + k) * 2 + 1];
+      ViewTerms t{};
+      if (FAN) {
+        t.d0 = -c1;
+        t.d1 = c0;
+        t.srx = c0 * (-sid);
+        t.sry = c1 * (-sid);
+        const float cpx = fmaf(c0, sdd, t.srx), cpy = fmaf(c1, sdd, t.sry);
+        const float p4x = cpx + t.d0, p4y = cpy + t.d1;
+        t.b = cpy - p4y;
+        t.d = cpx - p4x;
+        t.g = fmaf(-cpy, p4x, cpx * p4y);
+      } else {
+        t.srx = c0;
+        t.sry = -c1;
+      }
+      terms[k] = t;
+    }
+    __syncthreads();
+#pragma unroll 4  // four views in flight: a lane's chain per view is long and its load exposed
+    for (int k = 0; k < nv; ++k, base += (size_t)row_len(det) * sizeof(TS)) {
+      if (FAN) {
+        const ViewTerms t = terms[k];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          float s, dw;
+          fan_pixel<FAST>(t, pcx, pcy[p], s, dw);
+          const float f = sample_row<TS>(base, fdet, div_spacing<DIV>(s - do_, ds, ids));
+          val[p] = fmaf(f * dw, dw, val[p]);
+        }
+      } else {
+        const float c0 = terms[k].srx, m1 = pcx * terms[k].sry;
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          val[p] += sample_row<TS>(base, fdet, div_spacing<DIV>(fmaf(pcy[p], c0, m1) - do_, ds, ids));
+      }
+    }
+  }
+}
+
+// P pixels per lane, 16 rows apart; a block covers 16 x 16 P pixels.  FAST holds when the
+// detector spacing lies in [2^-30, 2^30] and every length of the geometry below 2^20 mm: the
+// denominator (at least 1e-6 where it is used) and the quotients then stay far inside the
+// range of the refined division, and a quotient so small that its residual is inexact
+// vanishes in the sampler's + 0.5.  The choices are uniform over the block and change no bit.
+template <typename TS, bool FAN, int P>
+__global__ void __launch_bounds__(256)
+back2d_rows_kernel(const TS *__restrict__ rows, float *__restrict__ vol, const float *__restrict__ rays,
+                   const float *__restrict__ vorigin, const float *__restrict__ dorigin,
+                   const float *__restrict__ vspacing, const float *__restrict__ dspacing,
+                   const float *__restrict__ sid_p, const float *__restrict__ sdd_p, int H, int W, int n, int det) {
+  __shared__ ViewTerms terms[kBackViews];
+  const int x = blockIdx.x * 16 + (threadIdx.x & 15);
+  const int y = blockIdx.y * 16 * P + (threadIdx.x >> 4);
+  const int b = blockIdx.z;
+  const float sx = vspacing[b * 2 + 1], sy = vspacing[b * 2 + 0];
+  const float ox = vorigin[b * 2 + 1], oy = vorigin[b * 2 + 0];
+  const float do_ = dorigin[b], ds = dspacing[b];
+  const float pcx = i2p((float)x, ox, sx);
+  float pcy[P], val[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    pcy[p] = i2p((float)(y + 16 * p), oy, sy);
+    val[p] = 0.0f;
+  }
+  const float *rb = rays + (size_t)b * n * 2;
+  rows += (size_t)b * n * row_len(det);
+  float sid = 0.0f, sdd = 0.0f;
+  if (FAN) {  // the parallel op passes no source distances
+    sid = sid_p[b];
+    sdd = sdd_p[b];
+  }
+  const float pow2 = pow2_reciprocal(ds);
+  const float far = fmaxf(fmaxf(fabsf(sid), fabsf(sdd)),
+                          fmaxf(fmaxf(fabsf(ox), fabsf(i2p((float)(W + 16), ox, sx))),
+                                fmaxf(fabsf(oy), fabsf(i2p((float)(H + 16 * P), oy, sy)))));
+  const bool fast = ds >= 0x1p-30f && ds <= 0x1p30f && far < 0x1p20f;
+  if (!fast)
+    back2d_rows<TS, FAN, false, kDivIeee, P>(rows, rb, n, det, pcx, pcy, do_, ds, 0.0f, sid, sdd, terms, val);
+  else if (pow2 != 0.0f)
+    back2d_rows<TS, FAN, true, kDivPow2, P>(rows, rb, n, det, pcx, pcy, do_, ds, pow2, sid, sdd, terms, val);
+  else
+    back2d_rows<TS, FAN, true, kDivRefine, P>(rows, rb, n, det, pcx, pcy, do_, ds, 1.0f / ds, sid, sdd, terms, val);
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    if (x < W && y + 16 * p < H) {
+      float *o = vol + ((size_t)b * H + (y + 16 * p)) * W + x;
+      *o = FAN ? (((sid * sdd) * kPi) * val[p]) / (float)n : (kPi * val[p]) / (float)n;
+    }
+  }
+}
+
 // rays per launch below which a ray gets four lanes
 constexpr long long kQuadRayLimit = 131072;
 
@@ -757,17 +942,57 @@ static int launch_proj2d(const char *name, const void *volume, int dtype, int ba
   return PYRONN_OK;
 }
 
+template <typename TS, bool FAN>
+static void launch_rows(const void *sino, int batch, int n, int det, const float *vo, const float *dor,
+                        const float *vs, const float *ds, const float *sid, const float *sdd, const float *rays, int H,
+                        int W, float *vol, void *ws, hipStream_t s) {
+  TS *rows = (TS *)ws;
+  const long long nrows = (long long)batch * n;
+  build_rows_kernel<TS><<<dim3((unsigned)((row_len(det) + 255) / 256), (unsigned)(nrows < 32768 ? nrows : 32768)),
+                          dim3(256), 0, s>>>((const TS *)sino, rows, det, nrows);
+  // One pixel per lane while the blocks fit the device at once (8 of 256 lanes per CU), two
+  // beyond: a few blocks past a full round run alone for as long as the round did (6 fan images
+  // of 301 x 277, 2052 blocks: 264 against 184 us; 8 of 512^2, 8192 blocks: 821 against 805),
+  // below it the second pixel only lengthens a block (512^2, 1024 blocks: 133 against 148).
+  const long long blocks = (long long)((W + 15) / 16) * ((H + 15) / 16) * batch;
+  if (blocks <= 2048) {
+    const dim3 grid((W + 15) / 16, (H + 15) / 16, batch);
+    back2d_rows_kernel<TS, FAN, 1><<<grid, dim3(256), 0, s>>>(rows, vol, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det);
+  } else {
+    const dim3 grid((W + 15) / 16, (H + 31) / 32, batch);
+    back2d_rows_kernel<TS, FAN, 2><<<grid, dim3(256), 0, s>>>(rows, vol, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det);
+  }
+}
+
 template <bool FAN>
 static int launch_back2d(const char *name, const void *sino, int dtype, int batch, int n, int det,
                          const float *vo, const float *dor, const float *vs, const float *ds,
                          const float *sid, const float *sdd, const float *rays, int H, int W,
-                         float *vol, hipStream_t s) {
+                         float *vol, void *ws, size_t ws_bytes, bool use_ws, hipStream_t s) {
   clear_error();
   PYRONN_CHECK_ARG(sino && vo && dor && vs && ds && rays && vol, "%s: null pointer", name);
   PYRONN_CHECK_ARG(!FAN || (sid && sdd), "%s: null source distances", name);
   PYRONN_CHECK_ARG(dtype_ok(dtype), "%s: bad dtype %d", name, dtype);
   PYRONN_CHECK_ARG(batch > 0 && batch <= 65535 && H > 0 && W > 0 && n > 0 && det > 0,
                    "%s: bad shape B=%d H=%d W=%d n=%d det=%d", name, batch, H, W, n, det);
+  if (use_ws) {
+    const size_t need = pyronn_backprojection2d_workspace_size(batch, n, det, dtype);
+    PYRONN_CHECK_ARG(need > 0, "%s: no bordered copy of %d detector pixels", name, det);
+    PYRONN_CHECK_ARG(ws != nullptr, "%s: null workspace", name);
+    PYRONN_CHECK_ARG(((uintptr_t)ws & 15) == 0, "%s: workspace must be 16-byte aligned", name);
+    if (ws_bytes < need) {
+      set_error("%s: workspace %zu bytes < required %zu", name, ws_bytes, need);
+      return PYRONN_ERR_WORKSPACE;
+    }
+    if (dtype == PYRONN_F32)
+      launch_rows<float, FAN>(sino, batch, n, det, vo, dor, vs, ds, sid, sdd, rays, H, W, vol, ws, s);
+    else if (dtype == PYRONN_BF16)
+      launch_rows<bf16s, FAN>(sino, batch, n, det, vo, dor, vs, ds, sid, sdd, rays, H, W, vol, ws, s);
+    else
+      launch_rows<_Float16, FAN>(sino, batch, n, det, vo, dor, vs, ds, sid, sdd, rays, H, W, vol, ws, s);
+    PYRONN_CHECK_LAUNCH(name);
+    return PYRONN_OK;
+  }
   dim3 grid((W + 15) / 16, (H + 15) / 16, batch);
   if (dtype == PYRONN_F32)
     back2d_kernel<float, FAN><<<grid, dim3(256), 0, s>>>((const float *)sino, vol, rays, vo, dor, vs, ds,
@@ -859,7 +1084,7 @@ extern "C" int pyronn_parallel_backprojection2d(const void *sinogram, int sinogr
                                                 float *volume, pyronn_stream_t stream) {
   return launch_back2d<false>("parallel_backprojection2d", sinogram, sinogram_dtype, batch, n_views,
                               det, volume_origin, detector_origin, volume_spacing,
-                              detector_spacing, nullptr, nullptr, ray_vectors, H, W, volume,
+                              detector_spacing, nullptr, nullptr, ray_vectors, H, W, volume, nullptr, 0, false,
                               (hipStream_t)stream);
 }
 
@@ -875,5 +1100,34 @@ extern "C" int pyronn_fan_backprojection2d(const void *sinogram, int sinogram_dt
   return launch_back2d<true>("fan_backprojection2d", sinogram, sinogram_dtype, batch, n_views, det,
                              volume_origin, detector_origin, volume_spacing, detector_spacing,
                              source_2_isocenter_distance, source_2_detector_distance,
-                             central_ray_vectors, H, W, volume, (hipStream_t)stream);
+                             central_ray_vectors, H, W, volume, nullptr, 0, false, (hipStream_t)stream);
+}
+
+extern "C" size_t pyronn_backprojection2d_workspace_size(int batch, int n_views, int det, int sinogram_dtype) {
+  if (batch <= 0 || n_views <= 0 || det <= 0 || !dtype_ok(sinogram_dtype)) return 0;
+  if (det >= (1 << 22)) return 0;  // the offset's float form (sample_row)
+  return align_up((size_t)batch * n_views * row_len(det) * dtype_bytes(sinogram_dtype), 256);
+}
+
+extern "C" int pyronn_parallel_backprojection2d_ws(const void *sinogram, int sinogram_dtype, int batch, int n_views,
+                                                   int det, const float *volume_origin, const float *detector_origin,
+                                                   const float *volume_spacing, const float *detector_spacing,
+                                                   const float *ray_vectors, int H, int W, float *volume,
+                                                   void *workspace, size_t workspace_bytes, pyronn_stream_t stream) {
+  return launch_back2d<false>("parallel_backprojection2d_ws", sinogram, sinogram_dtype, batch, n_views, det,
+                              volume_origin, detector_origin, volume_spacing, detector_spacing, nullptr, nullptr,
+                              ray_vectors, H, W, volume, workspace, workspace_bytes, true, (hipStream_t)stream);
+}
+
+extern "C" int pyronn_fan_backprojection2d_ws(const void *sinogram, int sinogram_dtype, int batch, int n_views, int det,
+                                              const float *volume_origin, const float *detector_origin,
+                                              const float *volume_spacing, const float *detector_spacing,
+                                              const float *source_2_isocenter_distance,
+                                              const float *source_2_detector_distance,
+                                              const float *central_ray_vectors, int H, int W, float *volume,
+                                              void *workspace, size_t workspace_bytes, pyronn_stream_t stream) {
+  return launch_back2d<true>("fan_backprojection2d_ws", sinogram, sinogram_dtype, batch, n_views, det, volume_origin,
+                             detector_origin, volume_spacing, detector_spacing, source_2_isocenter_distance,
+                             source_2_detector_distance, central_ray_vectors, H, W, volume, workspace,
+                             workspace_bytes, true, (hipStream_t)stream);
 }

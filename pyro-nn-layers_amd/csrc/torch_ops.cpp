@@ -216,20 +216,28 @@ at::Tensor back2d(bool fan, const at::Tensor &sinogram, at::IntArrayRef volume_s
   const int dt = dtype_code(sino, op);
   at::Tensor out = at::empty({B, H, W}, sino.options().dtype(at::kFloat));
   if (empty_output(out)) return out;
+  // the bordered copy of the projections that the backprojection samples
+  const size_t ws = pyronn_backprojection2d_workspace_size((int)B, (int)n, (int)det, dt);
+  at::Tensor work;
+  if (ws) work = at::empty({(int64_t)ws}, sino.options().dtype(at::kByte));
+  const float *vop = g.vo.data_ptr<float>(), *dop = g.dor.data_ptr<float>(), *vsp = g.vs.data_ptr<float>(),
+              *dsp = g.ds.data_ptr<float>(), *rp = g.rays.data_ptr<float>();
+  const float *sidp = fan ? g.sid.data_ptr<float>() : nullptr, *sddp = fan ? g.sdd.data_ptr<float>() : nullptr;
+  float *outp = out.data_ptr<float>();
+  const pyronn_stream_t st = cur_stream(sino);
   int rc;
-  if (fan)
-    rc = pyronn_fan_backprojection2d(sino.data_ptr(), dt, (int)B, (int)n, (int)det,
-                                     g.vo.data_ptr<float>(), g.dor.data_ptr<float>(),
-                                     g.vs.data_ptr<float>(), g.ds.data_ptr<float>(),
-                                     g.sid.data_ptr<float>(), g.sdd.data_ptr<float>(),
-                                     g.rays.data_ptr<float>(), (int)H, (int)W,
-                                     out.data_ptr<float>(), cur_stream(sino));
+  if (ws && fan)
+    rc = pyronn_fan_backprojection2d_ws(sino.data_ptr(), dt, (int)B, (int)n, (int)det, vop, dop, vsp, dsp, sidp, sddp,
+                                        rp, (int)H, (int)W, outp, work.data_ptr(), ws, st);
+  else if (ws)
+    rc = pyronn_parallel_backprojection2d_ws(sino.data_ptr(), dt, (int)B, (int)n, (int)det, vop, dop, vsp, dsp, rp,
+                                             (int)H, (int)W, outp, work.data_ptr(), ws, st);
+  else if (fan)
+    rc = pyronn_fan_backprojection2d(sino.data_ptr(), dt, (int)B, (int)n, (int)det, vop, dop, vsp, dsp, sidp, sddp, rp,
+                                     (int)H, (int)W, outp, st);
   else
-    rc = pyronn_parallel_backprojection2d(sino.data_ptr(), dt, (int)B, (int)n, (int)det,
-                                          g.vo.data_ptr<float>(), g.dor.data_ptr<float>(),
-                                          g.vs.data_ptr<float>(), g.ds.data_ptr<float>(),
-                                          g.rays.data_ptr<float>(), (int)H, (int)W,
-                                          out.data_ptr<float>(), cur_stream(sino));
+    rc = pyronn_parallel_backprojection2d(sino.data_ptr(), dt, (int)B, (int)n, (int)det, vop, dop, vsp, dsp, rp,
+                                          (int)H, (int)W, outp, st);
   check_rc(rc, op);
   return out;
 }

@@ -83,12 +83,13 @@ class _Plan(Capturable):
     def footprint(self) -> int:
         """Device bytes of one in-flight request: its input, the filtered copy, the GEMM
         filter's workspace (two float32 copies) if that filter is used, the detector cells
-        of the cone backprojection (four values per pixel) and the float32 output."""
+        of the cone backprojection (four values per pixel) or the planar one's copy, and the
+        float32 output."""
         nin = int(np.prod(self.input_shape))
         nout = int(np.prod(self.output_shape))
         e = torch.tensor([], dtype=self.storage).element_size()
         ws = 8 if self.filter_impl == "gemm" else 0
-        cells = 4 * e if isinstance(self, ConeFDK) else 0
+        cells = 4 * e if isinstance(self, ConeFDK) else e
         return nin * (e + e + ws + cells) + nout * 4
 
     def ramp_matrix(self) -> torch.Tensor:

@@ -60,6 +60,11 @@ _SIGS = {
                                         _vp, _vp, _sz, _vp]),
     "pyronn_fan_backprojection2d": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,
                                          _vp, _vp]),
+    "pyronn_backprojection2d_workspace_size": (_sz, [_i, _i, _i, _i]),
+    "pyronn_parallel_backprojection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp,
+                                                 _vp, _sz, _vp]),
+    "pyronn_fan_backprojection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,
+                                            _vp, _vp, _sz, _vp]),
     "pyronn_cone_projection3d_batched_workspace_size": (_sz, [_vp, _i, _i]),
     "pyronn_cone_projection3d_batched": (_i, [_vp, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "pyronn_cone_backprojection3d_batched_workspace_size": (_sz, [_vp, _i, _i]),

@@ -120,7 +120,10 @@ class FanProjector(Capturable):
 
     def footprint(self) -> int:
         e = torch.tensor([], dtype=self.storage).element_size()
-        return int(np.prod(self.input_shape)) * e + int(np.prod(self.output_shape)) * 4 + self.g.n_views * 8
+        H, W = self.g.volume_shape
+        pairs = (W + 4) * (H + 3) * 2 * e                    # the forward's pair copy
+        return (int(np.prod(self.input_shape)) * e + pairs + int(np.prod(self.output_shape)) * 4
+                + self.g.n_views * 8)
 
     def __call__(self, image: torch.Tensor) -> torch.Tensor:
         image = self._check_input(image)
@@ -151,7 +154,10 @@ class ParallelProjector(Capturable):
 
     def footprint(self) -> int:
         e = torch.tensor([], dtype=self.storage).element_size()
-        return int(np.prod(self.input_shape)) * e + int(np.prod(self.output_shape)) * 4 + self.g.n_views * 8
+        H, W = self.g.volume_shape
+        pairs = (W + 4) * (H + 3) * 2 * e                    # the forward's pair copy
+        return (int(np.prod(self.input_shape)) * e + pairs + int(np.prod(self.output_shape)) * 4
+                + self.g.n_views * 8)
 
     def __call__(self, image: torch.Tensor) -> torch.Tensor:
         image = self._check_input(image)

@@ -1,5 +1,6 @@
 // Test kit: exhaustive device checks of the library's arithmetic shortcuts:
 //  * rcp_rn() against the IEEE division 1.0f / w;
+//  * rcp_sqrt_fast() against 1.0f / sqrtf(t) over its range;
 //  * clamp_apron() (one v_med3_f32) against the clamp fminf(fmaxf(c, -1), n) that the
 //    oracle applies, with the reference value formed from the bit patterns by integer
 //    compares (so no compiler rewrite can turn it into the instruction under test).
@@ -50,7 +51,25 @@ __global__ void __launch_bounds__(256) clamp_check_kernel(unsigned *__restrict__
   counts[t] = bad;
 }
 
+// counts[t] = patterns t * 256 + k in rcp_sqrt_fast's range whose result differs from the
+// correctly rounded 1.0f / sqrtf(t).
+__global__ void __launch_bounds__(256) rcp_sqrt_check_kernel(unsigned *__restrict__ counts) {
+  const unsigned t = blockIdx.x * 256u + threadIdx.x;
+  unsigned bad = 0;
+  for (unsigned k = 0; k < 256u; ++k) {
+    const float w = __uint_as_float(t * 256u + k);
+    if (!pyronn::rcp_sqrt_ok(w)) continue;
+    bad += __float_as_uint(pyronn::rcp_sqrt_fast(w)) == __float_as_uint(1.0f / sqrtf(w)) ? 0u : 1u;
+  }
+  counts[t] = bad;
+}
+
 }  // namespace
+
+extern "C" int pyronn_testkit_rcp_sqrt_check(unsigned *counts, void *stream) {
+  hipLaunchKernelGGL(rcp_sqrt_check_kernel, dim3(65536), dim3(256), 0, (hipStream_t)stream, counts);
+  return (int)hipGetLastError();
+}
 
 extern "C" int pyronn_testkit_clamp_check(unsigned *counts, float n, void *stream) {
   hipLaunchKernelGGL(clamp_check_kernel, dim3(65536), dim3(256), 0, (hipStream_t)stream, counts, n);

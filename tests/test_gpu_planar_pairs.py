@@ -1,5 +1,6 @@
-"""The 2D projections through the pair copy of the images: the dispatch's edges (lanes per ray,
-remainders of the ray groups, spacings of each division, the largest copy) against the oracle."""
+"""The 2D projections through the pair copy of the images and the 2D backprojections through the
+bordered copy of the projections: the dispatch's edges (lanes per ray, remainders of the ray
+groups, pixels per lane, spacings of each division, the largest copy) against the oracle."""
 import math
 
 import numpy as np
@@ -76,3 +77,50 @@ def test_pairs_infinite_and_nan_pixels_reach_the_same_rays():
     for sp in ((0.25, 0.25), (1.0, 1.0), (0.3, 0.6)):
         got, ref = _run(False, img, sp, 40, 41, 0.5, 0.2, 0.0)
         assert np.array_equal(got, ref, equal_nan=True)
+
+
+def _back(fan, sino, shape, sp, ds, sid, storage=torch.float32, off=(0.0, 0.0)):
+    import pyronn_layers as pl
+    n, det = sino.shape[-2:]
+    org = (geo.centred_origin(shape, sp) + np.asarray(off)).astype(np.float32)
+    sp = np.asarray(sp, np.float32)
+    rays = geo.parallel_ray_vectors(n, 2 * math.pi).astype(np.float32)
+    do = np.float32(-(det - 1) / 2 * ds)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    x = dev(sino)[None].to(storage)
+    geom = [dev(org)[None], dev([[do]]), dev(sp)[None], dev([[ds]])]
+    s = x[0].float().cpu().numpy()
+    if fan:
+        out = pl.fan_backprojection2d(x, list(shape), *geom, dev([[sid]]), dev([[1.4 * sid]]), dev(rays)[None])
+        ref = orc.fan_backward(s, rays, shape, org, sp, do, np.float32(ds), sid=np.float32(sid),
+                               sdd=np.float32(1.4 * sid))
+    else:
+        out = pl.parallel_backprojection2d(x, list(shape), *geom, dev(rays)[None])
+        ref = orc.parallel_backward(s, rays, shape, org, sp, do, np.float32(ds))
+    return out[0].cpu().numpy(), ref[0] if isinstance(ref, tuple) else ref
+
+
+@pytest.mark.parametrize("fan", [False, True])
+@pytest.mark.parametrize("storage", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape, sp, n, det, ds", [
+    ((1, 1), (1.0, 1.0), 1, 1, 1.0),          # one pixel, one view, one detector pixel
+    ((17, 15), (0.7, 1.3), 7, 2, 9.0),        # a detector of one cell; refined division
+    ((33, 47), (1.0, 1.0), 129, 65, 0.5),     # one view past a block's table of 128
+    ((30, 31), (0.3, 0.3), 256, 40, 0.25),    # a detector smaller than the shadow
+    ((728, 730), (1.0, 1.0), 6, 911, 1.7),    # 2116 blocks: two pixels per lane, ragged rows
+    ((20, 20), (1.0, 1.0), 5, 30, 1e-12),     # a spacing outside the refined division's range
+])
+def test_rows_match_the_oracle(fan, storage, shape, sp, n, det, ds):
+    sino = np.random.default_rng(n + det).normal(size=(n, det)).astype(np.float32)
+    got, ref = _back(fan, sino, shape, sp, ds, 1.5 * max(shape[0] * sp[0], shape[1] * sp[1]), storage)
+    assert np.array_equal(got, ref, equal_nan=True), int((got != ref).sum())
+
+
+def test_rows_source_inside_the_image_and_far_lengths():
+    sino = np.random.default_rng(3).normal(size=(24, 50)).astype(np.float32)
+    # the source on pixels of the image: infinite weights and degenerate intersections
+    got, ref = _back(True, sino, (31, 31), (1.0, 1.0), 1.0, 10.0)
+    assert np.array_equal(got, ref, equal_nan=True)
+    # lengths of 2^20 mm and more take the IEEE sequences
+    got, ref = _back(True, sino, (31, 29), (1.0, 1.0), 1.0, 3.0e6, off=(1.1e6, 0.0))
+    assert np.array_equal(got, ref, equal_nan=True)
