@@ -68,35 +68,36 @@ __global__ void cone_setup_kernel(const float *__restrict__ P, const float *__re
 // z-fastest so that the 64 rays of a wave (16 detector rows ~ 16 neighbouring z
 // positions, and z is transverse to every ray of an orbit about the z axis) fall into few cache lines
 // for every view direction.  The zero border makes the reference's per-neighbour
-// bounds tests unnecessary.  Layout (xy quads): cell (x, y, z), x in [-1, W],
-// y in [-1, H], z in [-1, D + 1], holds [v(x,y,z), v(x+1,y,z), v(x,y+1,z), v(x+1,y+1,z)]
-// at index ((x+1) (H+2) + (y+1)) (D+3) + (z+1).  A sample needs the quads at z and
-// z + 1, which are adjacent:
-//  * f32 - 16-byte quads; a sample is two adjacent 16-byte loads sharing cache lines;
-//  * bf16 / f16 - 8-byte quads; a sample is one 16-byte load at 8-byte alignment.
-// Every storage type thus spends one quad per z step of a column: the 16-bit copy is
-// half the bytes of the f32 one.  (A 2x2x2 cell per z step for 16-bit storage, also one
-// 16-byte load per sample, occupies as many bytes as the f32 quads: on the 512^3 /
-// 720-view forward it took 473 ms against 389 ms for these quads in bf16, as the 16-bit
-// gathers are limited by L2 misses rather than by instruction issue.)
-// The build stages (x, z) tiles of two neighbouring y rows of the volume in LDS, so that
+// bounds tests unnecessary.  x in [-1, W], z in [-1, D + 1], columns of cells in (x, y) order:
+//  * f32 - x pairs, y in [-1, H + 1]: 8-byte cell (x, y, z) = [v(x,y,z), v(x+1,y,z)] at index
+//    ((x+1) (H+3) + (y+1)) (D+3) + (z+1).  The cells at z and z + 1 are adjacent, so a sample
+//    is two 16-byte loads at 8-byte alignment, from the columns of y and y + 1;
+//  * bf16 / f16 - xy quads, y in [-1, H]: 8-byte cell [v(x,y,z), v(x+1,y,z), v(x,y+1,z),
+//    v(x+1,y+1,z)] at index ((x+1) (H+2) + (y+1)) (D+3) + (z+1); a sample is one 16-byte load.
+// Every storage type thus spends 8 bytes per z step of a column.  Smaller cells pay through
+// the L1: f32 xy quads (16 bytes, the same two loads) took 378 ms on the 512^3 / 720-view
+// forward against 349 for x pairs (both at 16 x 16 pixel tiles; the quads were as fast with
+// any tile shape), and 16-bit 2x2x2 cells (16 bytes) 473 ms against 389 for the quads at the time.
+// The build stages (x, z) tiles of a cell's y rows (one or two) of the volume in LDS, so that
 // it reads the volume along x and writes the cells along z, both contiguously, with no
 // intermediate copy of the volume.
 // =====================================================================================
 template <typename TS> struct CellLayout {
-  static constexpr int kPerCell = 4;  // elements per cell (an xy quad)
-  static constexpr int kZExtra = 3;   // cells along z beyond D
+  static constexpr int kPerCell = sizeof(TS) == 4 ? 2 : 4;  // elements per cell (an x pair, an xy quad)
+  static constexpr int kYExtra = sizeof(TS) == 4 ? 3 : 2;   // rows of cells beyond H
+  static constexpr int kZExtra = 3;                         // cells along z beyond D
 };
 
 // The 16 bytes of the z and z + 1 quads of a 16-bit cell array: 8-byte aligned (the
 // target supports unaligned vector loads, so this stays one global_load_dwordx4).
 typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef float f32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 
 template <typename TS> static size_t cell_elems(int D, int H, int W) {
-  return (size_t)(W + 2) * (H + 2) * (D + CellLayout<TS>::kZExtra) * CellLayout<TS>::kPerCell;
+  return (size_t)(W + 2) * (H + CellLayout<TS>::kYExtra) * (D + CellLayout<TS>::kZExtra) * CellLayout<TS>::kPerCell;
 }
 
-// The four neighbours of a cell in one store: 16 bytes (f32) or 8 bytes (16-bit types).
+// Four neighbours in one store: 16 bytes (f32) or 8 bytes (16-bit types).
 __device__ __forceinline__ void store_cell(float *o, float a, float b, float c, float d) {
   *reinterpret_cast<float4 *>(o) = make_float4(a, b, c, d);
 }
@@ -114,9 +115,9 @@ __device__ __forceinline__ void store_cell(TS *o, TS a, TS b, TS c, TS d) {
 
 // One tile = cells (cx0 .. cx0 + 63, cy, cz0 .. cz0 + 31) in cell coordinates (voxel
 // x = cx - 1, y = cy - 1, z = cz - 1).  The block reads the voxels x = cx0 - 1 .. cx0 + 63
-// of rows y and y + 1 at the tile's 32 z positions into LDS (one wave row per (y, z),
-// contiguous in x; zero outside the volume), then writes each cell's quad, lanes along
-// z (32 consecutive 16- or 8-byte cells per half wave).  Tiles are numbered with cy
+// of row y (and y + 1 for quads) at the tile's 32 z positions into LDS (one wave row per
+// (y, z), contiguous in x; zero outside the volume), then writes each cell, lanes along
+// z (32 consecutive 8-byte cells per half wave).  Tiles are numbered with cy
 // fastest, so blocks running together read overlapping rows.
 constexpr int kCellTileX = 64, kCellTileZ = 32;
 
@@ -125,8 +126,9 @@ __global__ void __launch_bounds__(256)
 build_cells_kernel(const TS *__restrict__ vol, TS *__restrict__ cells, int W, int H, int D,
                    int batch) {
   using L = CellLayout<TS>;
-  __shared__ TS t[2][kCellTileZ][kCellTileX + 1];
-  const int Wc = W + 2, Hc = H + 2, Dc = D + L::kZExtra;
+  constexpr int kRowsY = L::kPerCell / 2;  // y rows of a cell
+  __shared__ TS t[kRowsY][kCellTileZ][kCellTileX + 1];
+  const int Wc = W + 2, Hc = H + L::kYExtra, Dc = D + L::kZExtra;
   const long long ntx = (Wc + kCellTileX - 1) / kCellTileX, ntz = (Dc + kCellTileZ - 1) / kCellTileZ;
   const long long tiles = ntx * ntz * Hc * batch;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -141,7 +143,7 @@ build_cells_kernel(const TS *__restrict__ vol, TS *__restrict__ cells, int W, in
     const TS *v = vol + (size_t)b * vstride;
     // 64 rows of (y, z): wave w loads rows w, w + 4, ...; lane l loads voxel x = cx0 - 1 + l,
     // lane 0 also the 65th voxel x = cx0 + 63
-    for (int row = wave; row < 2 * kCellTileZ; row += 4) {
+    for (int row = wave; row < kRowsY * kCellTileZ; row += 4) {
       const int ry = row / kCellTileZ, rz = row % kCellTileZ;
       const int y = cy - 1 + ry, z = cz0 - 1 + rz;
       const bool yz_in = y >= 0 && y < H && z >= 0 && z < D;
@@ -162,7 +164,10 @@ build_cells_kernel(const TS *__restrict__ vol, TS *__restrict__ cells, int W, in
       const int cx = cx0 + i;
       if (cx < Wc && cz < Dc) {
         TS *o = cells + ((((size_t)b * Wc + cx) * Hc + cy) * Dc + cz) * L::kPerCell;
-        store_cell(o, t[0][j][i], t[0][j][i + 1], t[1][j][i], t[1][j][i + 1]);
+        if constexpr (sizeof(TS) == 4)
+          *reinterpret_cast<float2 *>(o) = make_float2(t[0][j][i], t[0][j][i + 1]);
+        else
+          store_cell(o, t[0][j][i], t[0][j][i + 1], t[1][j][i], t[1][j][i + 1]);
       }
     }
     __syncthreads();
@@ -191,8 +196,8 @@ __device__ __forceinline__ void unpack2(uint32_t w, _Float16, float &a, float &b
 // operand exactly inside the FMA, one rounding as before), so a load costs no
 // conversions at all.
 // IT is the index type of the cell array: int for arrays within the 32-bit limits of
-// fwd_small_index, long long beyond them.  The 16-bit streamed march also takes
-// IT = unsigned: 32-bit byte offsets from a biased base (locate16, fwd_byte_offsets).
+// fwd_small_index, long long beyond them, and unsigned, 32-bit byte offsets from a biased
+// base (locate16), within those of fwd_byte_offsets.
 template <typename IT> struct CellKey { typedef unsigned type; };
 template <> struct CellKey<long long> { typedef unsigned long long type; };
 
@@ -211,6 +216,17 @@ template <typename IT> struct CellRegs<_Float16, IT> {
   }
 };
 
+// The address locate16's cell keys count from: the cell array itself, or for IT = unsigned
+// (byte offsets) the array moved by 8 HDc - 0x4B000000 bytes (wrapping 64-bit arithmetic;
+// every load adds the offset back).
+template <typename TS, typename IT>
+__device__ __forceinline__ const char *cell_base(const TS *cells, IT HDc) {
+  if constexpr (std::is_same<IT, unsigned>::value)
+    return reinterpret_cast<const char *>(cells) + (8ll * HDc - 0x4B000000ll);
+  else
+    return reinterpret_cast<const char *>(cells);
+}
+
 // Trilinear sample at (px, py, pz), lerp z -> y -> x exactly as
 // cone_projector_3D_CudaKernel.cu.cc:74-82.  With CLAMP the coordinate is clamped into
 // the zero border first (identical results for every finite coordinate); without it the
@@ -222,6 +238,7 @@ template <typename IT> struct CellRegs<_Float16, IT> {
 //    count below 2^31).
 //  * IT = long long: 64-bit integer products, for any volume whose sides are below 2^24
 //    (so that every coordinate and its floor are exact floats).
+//  * IT = unsigned: 32-bit byte offsets from a biased base (locate16, fwd_byte_offsets).
 template <typename TS, bool CLAMP, typename IT>
 __device__ __forceinline__ float sample_cells(const TS *__restrict__ cells, IT Dc, IT HDc,
                                               float px, float py, float pz, float fW, float fH,
@@ -234,7 +251,11 @@ __device__ __forceinline__ float sample_cells(const TS *__restrict__ cells, IT D
   const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
   const float xd = px - fx, yd = py - fy, zd = pz - fz;
   typename CellKey<IT>::type cell;
-  if constexpr (sizeof(IT) == 4) {
+  if constexpr (std::is_same<IT, unsigned>::value) {
+    const float yz = fmaf(fy, (float)Dc, fz);  // byte offset from a biased base, as in locate16
+    const float m = fmaf(yz, 8.0f, 0x1p23f + (float)(8u * (Dc + 1u)));
+    cell = (unsigned)__mul24((int)fx, (int)(8u * HDc)) + __float_as_uint(m);
+  } else if constexpr (sizeof(IT) == 4) {
     const int yz = (int)fmaf(fy, (float)Dc, fz);
     cell = (unsigned)(__mul24((int)fx, HDc) + yz + (HDc + Dc + 1));
   } else {
@@ -244,10 +265,18 @@ __device__ __forceinline__ float sample_cells(const TS *__restrict__ cells, IT D
   if (cell != r.cell) {
     r.cell = cell;
     if constexpr (sizeof(TS) == 4) {
-      const float4 *c4 = reinterpret_cast<const float4 *>(cells) + cell;
-      const float4 a = c4[0], b = c4[1];  // quads at z and z + 1
-      r.c[0] = a.x; r.c[1] = a.y; r.c[2] = a.z; r.c[3] = a.w;
-      r.c[4] = b.x; r.c[5] = b.y; r.c[6] = b.z; r.c[7] = b.w;
+      // x pairs at z and z + 1 of rows y and y + 1, one row of cells apart
+      const char *p0 = cell_base<TS, IT>(cells, HDc), *p1 = p0 + 8ll * Dc;
+      f32x4_a8 a, b;
+      if constexpr (std::is_same<IT, unsigned>::value) {
+        a = *reinterpret_cast<const f32x4_a8 *>(p0 + cell);
+        b = *reinterpret_cast<const f32x4_a8 *>(p1 + cell);
+      } else {
+        a = *reinterpret_cast<const f32x4_a8 *>(p0 + 8ll * cell);
+        b = *reinterpret_cast<const f32x4_a8 *>(p1 + 8ll * cell);
+      }
+      r.c[0] = a.x; r.c[1] = a.y; r.c[2] = b.x; r.c[3] = b.y;
+      r.c[4] = a.z; r.c[5] = a.w; r.c[6] = b.z; r.c[7] = b.w;
     } else {
       // quads at z and z + 1: words 0, 1 and 2, 3
       const u32x4_a8 q = *reinterpret_cast<const u32x4_a8 *>(reinterpret_cast<const uint2 *>(cells) + cell);
@@ -370,17 +399,6 @@ __device__ __forceinline__ void locate16(float px, float py, float pz, IT Dc, IT
     cell = (unsigned long long)((long long)(int)fx * HDc + (long long)(int)fy * Dc + (long long)(int)fz +
                                 (HDc + Dc + 1));
   }
-}
-
-// The address locate16's cell keys count from: the cell array itself, or for IT = unsigned
-// (byte offsets) the array moved by 8 HDc - 0x4B000000 bytes (wrapping 64-bit arithmetic;
-// every load adds the offset back).
-template <typename TS, typename IT>
-__device__ __forceinline__ const char *cell_base(const TS *cells, IT HDc) {
-  if constexpr (std::is_same<IT, unsigned>::value)
-    return reinterpret_cast<const char *>(cells) + (8ll * HDc - 0x4B000000ll);
-  else
-    return reinterpret_cast<const char *>(cells);
 }
 
 template <typename IT, typename K>
@@ -592,16 +610,19 @@ __device__ __forceinline__ float march_ray(const TS *__restrict__ v, IT Dc, IT H
 // (z-neighbours in one z-fastest cell column, mostly one line) rather than four columns
 // (up to four different cell columns).
 // Work order: workgroups are dispatched round-robin over the 8 XCDs, so block id
-// b runs on XCD b % 8.  XCD k takes detector tile rows k, k+8, k+16, ...; within a
-// tile row it walks tiles (outer) and views (inner).  The blocks resident on one XCD
-// at any time are therefore one or two 16 x 16 tiles of one 16-row band over a few
-// hundred consecutive views: their rays cross the same z slab of the volume, and the
-// rays of one pixel in consecutive views are half a degree apart, so lines fetched
-// for one view are read again by the next while they are still in that XCD's L2.
-// (Measured on the 512^3 / 720-view forward against views outer, tiles inner: 483
-// against 534 ms in f32, 328 against 390 ms in bf16; groups of 2 to 32 tiles per pass
-// over the views fell in between, the fewer tiles the faster.)  The order changes
-// only which lane computes which ray, never the arithmetic of a ray.
+// b runs on XCD b % 8.  The detector tiles, row by row, are dealt to the XCDs in turn, and
+// an XCD walks its tiles (outer) and views (inner).  The blocks resident on one XCD at any
+// time are therefore one or two 16 x 16 tiles over a few hundred consecutive views: the rays
+// of one pixel in consecutive views are half a degree apart, so lines fetched for one view
+// are read again by the next while they are still in that XCD's L2; all XCDs work on
+// neighbouring tiles of one row, whose rays cross the same z slab of the volume, so what one
+// XCD fetches from memory the others find in the cache behind the L2s; and every XCD has the
+// same number of tiles to within one, of every kind.  (Measured against whole tile rows dealt
+// to the XCDs, which also left an XCD with up to twice the mean on detectors of few rows: f32
+// 512^3 / 720 views 350 -> 333 ms, 384^3 59.5 -> 56.4, 256^3 / 400^2 detector 28.4 -> 22.7,
+// 128^3 2.06 -> 1.72; bf16 256^3 21.8 -> 17.9, 512^3 equal.  Views outer, tiles inner took
+// 534 ms where tiles outer took 483.)  The order changes only which lane computes which ray,
+// never the arithmetic of a ray.
 // Ray setup: cone_projector_3D_CudaKernel.cu.cc:197-221; march: :87-181
 // (hardware_interp: cone_projector_3D_CudaKernel_hardware_interp.cu.cc:43-142).
 // =====================================================================================
@@ -635,14 +656,12 @@ template <typename TS, bool HW, typename IT, bool DIRECT = false, typename TL = 
 __device__ __forceinline__ void fwd_block(const FwdProblem &P, long long q) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int xcd = (int)(q % kXcds);
-  const long long qq = q / kXcds;
-  const long long per_row = (long long)P.n * P.tiles_x;
-  const int band = (int)(qq / per_row);
-  const int ty = band * kXcds + xcd;
-  if (ty >= P.tiles_y) return;
-  const long long w_ = qq - (long long)band * per_row;
-  const int tx = (int)(w_ / P.n);
-  const int view = (int)(w_ - (long long)tx * P.n);
+  const long long qq = q / kXcds;  // view fastest, then the XCD's tiles
+  const long long k = qq / P.n;
+  const int view = (int)(qq - k * P.n);
+  const long long t = k * kXcds + xcd;
+  if (t >= (long long)P.tiles_x * P.tiles_y) return;
+  const int ty = (int)(t / P.tiles_x), tx = (int)(t - (long long)ty * P.tiles_x);
   const int W = P.W, H = P.H, D = P.D, Hd = P.Hd, Wd = P.Wd;
   // Lanes past the detector's last column or row: in the 16-bit streamed march they march a
   // copy of the edge pixel's ray and store nothing, so that every lane of the wave takes
@@ -661,7 +680,7 @@ __device__ __forceinline__ void fwd_block(const FwdProblem &P, long long q) {
   const TS *v = static_cast<const TS *>(P.cells);
   // z-fastest cell strides, or the volume's row and plane strides (DIRECT)
   const IT Wp = DIRECT ? (IT)W : (IT)D + CellLayout<TS>::kZExtra;
-  const IT HWp = DIRECT ? (IT)H * W : (IT)(H + 2) * Wp;
+  const IT HWp = DIRECT ? (IT)H * W : (IT)(H + CellLayout<TS>::kYExtra) * Wp;
   const float fW = (float)W, fH = (float)H, fD = (float)D;
   float *out = P.sino + ((size_t)view * Hd + row) * (size_t)Wd + col;
   const float u = (float)col, w = (float)row;
@@ -1074,9 +1093,9 @@ __global__ void __launch_bounds__(256, 5) cone_bp_items_kernel(BpBatch B) {
 // =====================================================================================
 // Host side
 // =====================================================================================
-static size_t cell_elems_dt(int dtype, int D, int H, int W) {
-  return dtype == PYRONN_F32 ? cell_elems<float>(D, H, W) : cell_elems<bf16s>(D, H, W);
-}
+// Elements the workspace holds for the cells: four per cell of the 16-bit layout, for f32 too
+// (whose x pairs fill about half of them).
+static size_t cell_elems_dt(int, int D, int H, int W) { return cell_elems<bf16s>(D, H, W); }
 
 // Volumes the forward accepts: every side below 2^24 - 3, so that each cell coordinate and
 // its floor are exact floats (the reference indexes with uint32 and so takes volumes below
@@ -1088,16 +1107,15 @@ static bool fwd_volume_ok(int D, int H, int W) {
 // Whether the forward may use the 32-bit cell index (sample_cells, IT = int): fewer than 2^31
 // cells, and W + 2 and the (y, z) plane of cells below 2^23 for the 24-bit multiply and the
 // exact float FMA of the sampler.  Larger volumes take the 64-bit index.
-static bool fwd_small_index(int D, int H, int W) {
-  const long long cells = (long long)(W + 2) * (H + 2) * (D + CellLayout<float>::kZExtra);
-  return cells < (long long)INT32_MAX && W + 2 < (1 << 23) &&
-         (long long)(H + 2) * (D + CellLayout<float>::kZExtra) < (1LL << 23);
+template <typename TS> static bool fwd_small_index(int D, int H, int W) {
+  const long long plane = (long long)(H + CellLayout<TS>::kYExtra) * (D + CellLayout<TS>::kZExtra);
+  return (W + 2) * plane < (long long)INT32_MAX && W + 2 < (1 << 23) && plane < (1LL << 23);
 }
-// Whether the 16-bit forward may address its 8-byte cells by 32-bit byte offsets (locate16,
-// IT = unsigned): 8 (H + 2) Dc below 2^23 for the exact float and the 24-bit multiply, and
+// Whether the forward may address its 8-byte cells by 32-bit byte offsets (locate16,
+// IT = unsigned): 8 Hc Dc below 2^23 for the exact float and the 24-bit multiply, and
 // the cell array within 0xB5000000 bytes so that offset + 0x4B000000 stays below 2^32.
-static bool fwd_byte_offsets(int D, int H, int W) {
-  const long long plane = (long long)(H + 2) * (D + CellLayout<float>::kZExtra);
+template <typename TS> static bool fwd_byte_offsets(int D, int H, int W) {
+  const long long plane = (long long)(H + CellLayout<TS>::kYExtra) * (D + CellLayout<TS>::kZExtra);
   return W + 2 < (1 << 23) && 8 * plane < (1LL << 23) && 8 * (W + 2) * plane <= 0xB5000000LL;
 }
 static size_t det_cells(int n, int Hd, int Wd) { return (size_t)n * (Hd + 2) * (Wd + 2); }
@@ -1109,12 +1127,12 @@ static bool det_fidx(int Hd, int Wd) { return (long long)(Hd + 2) * (Wd + 2) <= 
 constexpr long long kMaxGridX = (1LL << 24) - 1;
 constexpr int kMaxGridYZ = 65535;
 
-// Blocks of one forward launch per batch item: 8 XCD lanes x tile-row bands x views x tiles
-// (tile shape `tile`, kFwdTiles).
+// Blocks of one forward launch per batch item: 8 XCDs x tiles of each x views (tile shape
+// `tile`, kFwdTiles).
 static long long fwd_blocks(int n, int Hd, int Wd, int tile = 0) {
   const int tc = fwd_tile_cols(tile), tr = fwd_tile_rows(tile);
   const long long tiles_x = (Wd + tc - 1) / tc, tiles_y = (Hd + tr - 1) / tr;
-  return (long long)kXcds * ((tiles_y + kXcds - 1) / kXcds) * n * tiles_x;
+  return (long long)kXcds * n * ((tiles_x * tiles_y + kXcds - 1) / kXcds);
 }
 // Views per forward launch (0: one view alone exceeds a launch).
 static int fwd_views_per_launch(int n, int Hd, int Wd, int tile = 0) {
@@ -1122,66 +1140,45 @@ static int fwd_views_per_launch(int n, int Hd, int Wd, int tile = 0) {
   return (int)(per < n ? per : n);
 }
 
-// Tile shape (kFwdTiles) of the single-problem forward with a cell copy: 32 x 8 pixels of
-// 8 x 8 waves for f32 cells, and for 16-bit cells of volumes up to 2^25 voxels; 16 x 16 of
-// 4 x 16 waves for larger 16-bit volumes.  Measured per problem (phantom volumes, 16 x 16 /
-// 4 x 16 against 32 x 8 / 8 x 8): f32 equal on the 512^3 / 720-view / 1024 x 768 workload
-// (372.7 / 372.9 ms) and 3-11% faster on the others (256^3 / 360 views / 400^2: 27.8 / 24.8
-// ms); bf16 faster up to 320^3 (43.8 / 41.0 ms), equal at 384^3 and slower beyond (512^3:
-// 213.2 / 237.6 ms).  The shape changes which lane computes which ray, never a result.
-template <typename TS> static int fwd_single_tile(int D, int H, int W) {
-  return (sizeof(TS) == 4 || (long long)D * H * W <= (1LL << 25)) ? 2 : 0;
-}
-
 template <typename TS>
 static void launch_cells(const void *vol, void *cells, int B, int D, int H, int W, hipStream_t stream) {
   const long long tiles = (long long)((W + 2 + kCellTileX - 1) / kCellTileX) *
-                          ((D + CellLayout<TS>::kZExtra + kCellTileZ - 1) / kCellTileZ) * (H + 2) * B;
+                          ((D + CellLayout<TS>::kZExtra + kCellTileZ - 1) / kCellTileZ) * (H + CellLayout<TS>::kYExtra) * B;
   const long long blocks = tiles < 65536 * 8 ? tiles : 65536 * 8;
   build_cells_kernel<TS><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>((const TS *)vol, (TS *)cells, W, H,
                                                                            D, B);
 }
 
 template <typename TS, typename IT>
-static void launch_fwd_it(bool hw, int tile, const FwdProblem &P, dim3 grid, long long cs, int n_all,
-                          hipStream_t stream) {
-  using T2 = FwdTile<32, 8, 8>;
-  if (tile == 2) {
-    if (hw)
-      cone_fwd_kernel<TS, true, IT, false, T2><<<grid, dim3(256), 0, stream>>>(P, cs, n_all);
-    else
-      cone_fwd_kernel<TS, false, IT, false, T2><<<grid, dim3(256), 0, stream>>>(P, cs, n_all);
-  } else if (hw) {
+static void launch_fwd_it(bool hw, const FwdProblem &P, dim3 grid, long long cs, int n_all, hipStream_t stream) {
+  if (hw)
     cone_fwd_kernel<TS, true, IT><<<grid, dim3(256), 0, stream>>>(P, cs, n_all);
-  } else {
+  else
     cone_fwd_kernel<TS, false, IT><<<grid, dim3(256), 0, stream>>>(P, cs, n_all);
-  }
 }
 
+// 16 x 16 pixel tiles of 4 x 16 waves for every storage and size.  Measured with x-pair f32 cells
+// (against 32 x 8 tiles of 8 x 8 waves, whole tile rows dealt to the XCDs in both): f32 512^3 350
+// / 379 ms, 384^3 58.5 / 63.2, 256^3 23.1 / 23.9, 192^3 9.6 / 10.2, 90^3 0.29 / 0.32; bf16 512^3
+// 246 / 262, 256^3 18.2 / 19.0, 192^3 7.75 / 8.05.
 template <typename TS>
 static void launch_fwd(bool hw, const void *cells, float *sino, const float *inv_ar,
                        const float *src, const float *step, const float *spacing, int B, int D,
                        int H, int W, int n, int Hd, int Wd, hipStream_t stream) {
   const long long cs = (long long)cell_elems<TS>(D, H, W);
-  const bool small = fwd_small_index(D, H, W);
-  const int tile = fwd_single_tile<TS>(D, H, W);
-  const int tc = fwd_tile_cols(tile), tr = fwd_tile_rows(tile);
-  const int per = fwd_views_per_launch(n, Hd, Wd, tile);
+  const bool small = fwd_small_index<TS>(D, H, W);
+  const int per = fwd_views_per_launch(n, Hd, Wd);
   for (int v0 = 0; v0 < n; v0 += per) {
     const int k = n - v0 < per ? n - v0 : per;
     FwdProblem P{cells, sino + (size_t)v0 * Hd * Wd, inv_ar + (size_t)v0 * 9, src + (size_t)v0 * 3, step,
-                 spacing, W, H, D, k, Hd, Wd, (Wd + tc - 1) / tc, (Hd + tr - 1) / tr, 0};
-    dim3 grid((unsigned)fwd_blocks(k, Hd, Wd, tile), 1, B);
-    if constexpr (sizeof(TS) == 2) {
-      if (fwd_byte_offsets(D, H, W)) {
-        launch_fwd_it<TS, unsigned>(hw, tile, P, grid, cs, n, stream);
-        continue;
-      }
-    }
-    if (small)
-      launch_fwd_it<TS, int>(hw, tile, P, grid, cs, n, stream);
+                 spacing, W, H, D, k, Hd, Wd, (Wd + 15) / 16, (Hd + 15) / 16, 0};
+    dim3 grid((unsigned)fwd_blocks(k, Hd, Wd), 1, B);
+    if (fwd_byte_offsets<TS>(D, H, W))
+      launch_fwd_it<TS, unsigned>(hw, P, grid, cs, n, stream);
+    else if (small)
+      launch_fwd_it<TS, int>(hw, P, grid, cs, n, stream);
     else
-      launch_fwd_it<TS, long long>(hw, tile, P, grid, cs, n, stream);
+      launch_fwd_it<TS, long long>(hw, P, grid, cs, n, stream);
   }
 }
 
@@ -1643,7 +1640,7 @@ static int fwd_batched(const pyronn_cone_problem *pr, int count, bool hw, int bp
   ws += kCounterBytes;
   FwdBatch fb{};
   long long begin = 0;
-  bool small = true, bytes = sizeof(TS) == 2;
+  bool small = true, bytes = true;
   const int tc = fwd_tile_cols(tile), tr = fwd_tile_rows(tile);
   for (int k = 0; k < count; ++k) {
     const pyronn_cone_problem &p = pr[k];
@@ -1654,8 +1651,8 @@ static int fwd_batched(const pyronn_cone_problem *pr, int count, bool hw, int bp
     cone_setup_kernel<<<dim3((p.n_views + 127) / 128), dim3(128), 0, s>>>(
         p.projection_matrices, p.volume_origin, p.volume_spacing, 1, p.n_views, inv_ar, src);
     launch_cells<TS>(p.input, cells, 1, p.D, p.H, p.W, s);
-    small = small && fwd_small_index(p.D, p.H, p.W);
-    bytes = bytes && fwd_byte_offsets(p.D, p.H, p.W);
+    small = small && fwd_small_index<TS>(p.D, p.H, p.W);
+    bytes = bytes && fwd_byte_offsets<TS>(p.D, p.H, p.W);
     fb.p[k] = FwdProblem{cells, p.output, inv_ar, src, p.step_size, p.volume_spacing,
                          p.W, p.H, p.D, p.n_views, p.det_h, p.det_w,
                          (p.det_w + tc - 1) / tc, (p.det_h + tr - 1) / tr, begin};
@@ -1672,12 +1669,10 @@ static int fwd_batched(const pyronn_cone_problem *pr, int count, bool hw, int bp
     reset_counters_kernel<<<1, 64, 0, s>>>(counters);
   }
   const dim3 g((unsigned)grid);
-  if constexpr (sizeof(TS) == 2) {
-    if (bytes) {
-      if (hw) launch_fwd_persistent<TS, true, unsigned>(fb, tile, g, counters, s);
-      else launch_fwd_persistent<TS, false, unsigned>(fb, tile, g, counters, s);
-      return PYRONN_OK;
-    }
+  if (bytes) {
+    if (hw) launch_fwd_persistent<TS, true, unsigned>(fb, tile, g, counters, s);
+    else launch_fwd_persistent<TS, false, unsigned>(fb, tile, g, counters, s);
+    return PYRONN_OK;
   }
   if (small) {
     if (hw) launch_fwd_persistent<TS, true, int>(fb, tile, g, counters, s);

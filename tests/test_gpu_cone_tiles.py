@@ -1,0 +1,31 @@
+"""How the cone kernels deal their tiles to the XCDs, at tile counts around the 8 XCDs, and the f32 forward's cell indexes at the limit of its 32-bit byte offsets, all
+against the oracle."""
+import pytest
+
+import gpu_helpers as gh
+from test_gpu_limits import _check_views, _orbit, _rand_volume
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("det", [(16, 16), (17, 113), (129, 16), (15, 128), (40, 152), (100, 50)])
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_forward_tiles_one_to_forty(det, storage):
+    shape = (20, 24, 18)
+    sp, og, P = _orbit(shape, 5, 100.0, 160.0, det, (60.0 / det[0], 60.0 / det[1]))
+    vol = _rand_volume(shape, det[0], gh.DT[storage][1])
+    _check_views(vol, P, sp, og, det, 0.5, False, views=range(5))
+
+
+@pytest.mark.parametrize("shape, fits", [
+    ((1000, 1019, 368), True),    # 3.034e9 bytes of x pairs, the last size within the byte offsets
+    ((1000, 1020, 368), False),   # one row more: the 32-bit cell index
+    ((1021, 1021, 2), False),     # 8 (H + 3)(D + 3) = 2^23
+])
+def test_forward_f32_cell_index_at_the_byte_offsets_limit(shape, fits):
+    plane = (shape[1] + 3) * (shape[0] + 3)
+    assert (8 * plane < 2 ** 23 and 8 * (shape[2] + 2) * plane <= 0xB5000000) == fits
+    det = (32, 48)
+    sp, og, P = _orbit(shape, 4, 3000.0, 5000.0, det, (30.0, 12.0 if shape[2] > 2 else 0.5))
+    print(f"f32 cells {shape}", flush=True)
+    _check_views(_rand_volume(shape, 7), P, sp, og, det, 0.5, False, views=(0, 1))
