@@ -1,8 +1,13 @@
-"""How the cone kernels deal their tiles to the XCDs, at tile counts around the 8 XCDs, and the f32 forward's cell indexes at the limit of its 32-bit byte offsets, all
+"""How the cone kernels deal their tiles to the XCDs, at tile counts around the 8 XCDs and the
+four strips, and the f32 forward's cell indexes at the limit of its 32-bit byte offsets, all
 against the oracle."""
+import numpy as np
 import pytest
+import torch
 
 import gpu_helpers as gh
+import oracle as orc
+from pyronn_layers import geometry as geo
 from test_gpu_limits import _check_views, _orbit, _rand_volume
 
 pytestmark = pytest.mark.gpu
@@ -15,6 +20,21 @@ def test_forward_tiles_one_to_forty(det, storage):
     sp, og, P = _orbit(shape, 5, 100.0, 160.0, det, (60.0 / det[0], 60.0 / det[1]))
     vol = _rand_volume(shape, det[0], gh.DT[storage][1])
     _check_views(vol, P, sp, og, det, 0.5, False, views=range(5))
+
+
+@pytest.mark.parametrize("plane", [(16, 16), (1, 80), (112, 33), (40, 150), (129, 65), (64, 64)])
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+def test_backprojection_tiles_one_to_forty(plane, storage):
+    shape = (11,) + plane
+    det = (24, 40)
+    sp = np.ones(3, np.float32)
+    og = geo.centred_origin(shape, sp).astype(np.float32)
+    P = geo.circular_projection_matrices(6, 300.0, 480.0, det, (1.5, 6.0)).astype(np.float32)
+    s = np.random.default_rng(plane[0]).normal(size=(6,) + det).astype(np.float32)
+    s = torch.tensor(s).to(gh.DT[storage][1]).float().numpy()
+    got = gh.cone_backward(s, P, sp, og, shape, storage=storage)[0]
+    ref, _ = orc.cone_backward(s, P, shape, sp, og)
+    assert np.array_equal(got, ref)
 
 
 @pytest.mark.parametrize("shape, fits", [
