@@ -4,8 +4,8 @@
 //   cone_setup_kernel   per-view FP64 geometry (M^-1, camera centre) on the device
 //   build_cells_kernel  copy of the volume as neighbourhood cells with a zero border
 //                       (what the forward sampler reads)
-//   build_det_cells_kernel  copy of the sinogram as 2x2 neighbourhood cells with a
-//                       zero border (what the backprojection sampler reads)
+//   build_det_cells_kernel  copy of the sinogram as row-pair cells with a zero border
+//                       (what the backprojection sampler reads)
 //   cone_fwd_kernel     ray-driven forward projection, one lane per detector pixel
 //   cone_bp_kernel      voxel-driven backprojection, one lane per ZPT voxels in z
 //
@@ -97,10 +97,7 @@ template <typename TS> static size_t cell_elems(int D, int H, int W) {
   return (size_t)(W + 2) * (H + CellLayout<TS>::kYExtra) * (D + CellLayout<TS>::kZExtra) * CellLayout<TS>::kPerCell;
 }
 
-// Four neighbours in one store: 16 bytes (f32) or 8 bytes (16-bit types).
-__device__ __forceinline__ void store_cell(float *o, float a, float b, float c, float d) {
-  *reinterpret_cast<float4 *>(o) = make_float4(a, b, c, d);
-}
+// The four 16-bit neighbours of a cell in one 8-byte store.
 template <typename TS>
 __device__ __forceinline__ void store_cell(TS *o, TS a, TS b, TS c, TS d) {
   static_assert(sizeof(TS) == 2, "16-bit storage");
@@ -833,12 +830,26 @@ __global__ void __launch_bounds__(256) cone_fwd_items_kernel(FwdBatch B, long lo
 }
 
 // =====================================================================================
-// Detector cells for the backprojection: per view, cell (u, v), u in [-1, W_d],
-// v in [-1, H_d], holds the bilinear neighbourhood
-//   [s(u,v), s(u+1,v), s(u,v+1), s(u+1,v+1)]
-// with zeros outside the detector, so one update is one 16-byte (f32) or 8-byte
-// (bf16 / f16) load.
+// Detector cells for the backprojection: per view, 2-element cell (u, v), u in [-1, W_d + 1],
+// v in [-1, H_d], u fastest, holds [s(u, v), s(u, v + 1)] with zeros outside the detector.  The
+// cells of u and u + 1 together are the bilinear neighbourhood, so one update is one load of
+// 16 bytes (f32) or 8 bytes (bf16 / f16) at cell alignment.  (With the whole neighbourhood in
+// each cell, twice the bytes through the L1 and L2 and in the build, the 512^3 / 720-view
+// backprojection took, build included, 64.0 against 53.6 ms in f32, 54.6 against 50.6 in bf16,
+// and 256^3 / 360 views 3.72 against 3.19 and 3.31 against 3.01.  A wave's load now takes 20
+// cycles of the address path, 16 at best; 8 x 8 waves and one wave per SIMD less change nothing.)
 // =====================================================================================
+template <typename TS> struct DetLoad {
+  typedef uint32_t raw __attribute__((ext_vector_type(2), aligned(4)));
+  static constexpr int kShift = 2;  // bytes of a cell, log2
+};
+template <> struct DetLoad<float> {
+  typedef f32x4_a8 raw;
+  static constexpr int kShift = 3;
+};
+__host__ __device__ inline int det_cols(int Wd) { return Wd + 3; }
+__host__ __device__ inline size_t det_image(int Hd, int Wd) { return (size_t)(Hd + 2) * det_cols(Wd); }
+
 template <typename TS>
 __device__ __forceinline__ TS pix(const TS *__restrict__ s, int u, int v, int Wd, int Hd) {
   if (u < 0 || u >= Wd || v < 0 || v >= Hd) return zero_of<TS>();
@@ -846,15 +857,15 @@ __device__ __forceinline__ TS pix(const TS *__restrict__ s, int u, int v, int Wd
 }
 
 // Lanes along a row of cells (x), blocks over runs of kDetCellRows cell rows (y) and
-// images (z), so no lane divides.  Walking down its column, a lane keeps the detector
-// row it read for the cell above and loads only the next row: two loads and one vector
-// store per cell, every cell written by exactly one lane.
+// images (z), so no lane divides.  Walking down its column, a lane keeps the pixel it read
+// for the cell above and loads only the next one: one load and one vector store per cell,
+// every cell written by exactly one lane.
 constexpr int kDetCellRows = 16;
 
 template <typename TS>
 __global__ void build_det_cells_kernel(const TS *__restrict__ sino, TS *__restrict__ cells,
                                        int Hd, int Wd, int images) {
-  const int Wc = Wd + 2, Hc = Hd + 2;
+  const int Wc = det_cols(Wd), Hc = Hd + 2;
   const int cu = blockIdx.x * blockDim.x + threadIdx.x;
   if (cu >= Wc) return;
   const int u = cu - 1;
@@ -862,29 +873,36 @@ __global__ void build_det_cells_kernel(const TS *__restrict__ sino, TS *__restri
     const TS *s = sino + (size_t)img * Hd * Wd;
     for (int cv0 = blockIdx.y * kDetCellRows; cv0 < Hc; cv0 += gridDim.y * kDetCellRows) {
       const int cv1 = cv0 + kDetCellRows < Hc ? cv0 + kDetCellRows : Hc;
-      TS *o = cells + (((size_t)img * Hc + cv0) * Wc + cu) * 4;
+      TS *o = cells + ((size_t)img * det_image(Hd, Wd) + (size_t)cv0 * Wc + cu) * 2;
       // cell row cv covers detector rows v = cv - 1 and v + 1 = cv
-      TS a = pix(s, u, cv0 - 1, Wd, Hd), b = pix(s, u + 1, cv0 - 1, Wd, Hd);
+      TS e[2] = {pix(s, u, cv0 - 1, Wd, Hd), zero_of<TS>()};
 #pragma unroll 4
-      for (int cv = cv0; cv < cv1; ++cv, o += (size_t)Wc * 4) {
-        const TS c = pix(s, u, cv, Wd, Hd), d = pix(s, u + 1, cv, Wd, Hd);
-        store_cell(o, a, b, c, d);
-        a = c;
-        b = d;
+      for (int cv = cv0; cv < cv1; ++cv, o += (size_t)Wc * 2) {
+        e[1] = pix(s, u, cv, Wd, Hd);
+        if constexpr (sizeof(TS) == 4) {
+          *reinterpret_cast<float2 *>(o) = make_float2(e[0], e[1]);
+        } else {
+          uint32_t w;
+          __builtin_memcpy(&w, e, 4);
+          *reinterpret_cast<uint32_t *>(o) = w;
+        }
+        e[0] = e[1];
       }
     }
   }
 }
 
 // Bilinear sample, lerp x then y (cone_backprojector_3D_CudaKernel.cu.cc:55-82),
-// zero outside the detector.
-// FIDX: img points at cell (0, 0) (not at the cell array's start, cell (-1, -1)) and the
-// host guarantees (H_d + 2)(W_d + 2) <= 2^24, so the cell offset fy W_c + fx is an integer
-// of magnitude below 2^24 that one float FMA forms exactly (two instructions fewer than
-// the integer form).
+// zero outside the detector.  img is the view's first cell, (-1, -1).
+// FIDX: the host guarantees (H_d + 2)(W_d + 3) < 2^23, so with the bias 2^23 the cell index is an
+// exact float in [2^23, 2^24) whose bits, shifted by the cell size, are a 32-bit byte offset from
+// an address moved by the shifted exponent bits: three instructions and a load from a uniform
+// base.
 template <typename TS, bool HW, bool FIDX>
 __device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, float u, float v,
                                             float fW, float fH) {
+  typedef typename DetLoad<TS>::raw raw;
+  constexpr int S = DetLoad<TS>::kShift;
   if (HW) {  // tex2DLayered(u + 0.5, v + 0.5, n)
     u = (u + 0.5f) - 0.5f;
     v = (v + 0.5f) - 0.5f;
@@ -893,16 +911,21 @@ __device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, 
   v = clamp_apron(v, fH);
   const float fx = floorf(u), fy = floorf(v);
   const float xd = u - fx, yd = v - fy;
-  // signed 24-bit multiply (full rate); the host keeps W_d + 2 and H_d + 2 below 2^23
-  const int c = FIDX ? (int)fmaf(fy, (float)Wc, fx) : __mul24((int)fy, Wc) + (int)fx + (Wc + 1);
+  raw q;
+  if constexpr (FIDX) {
+    const uint32_t at = __float_as_uint(fmaf(fy, (float)Wc, fx + (0x1p23f + (float)(Wc + 1)))) << S;
+    q = *reinterpret_cast<const raw *>(reinterpret_cast<const char *>(img) - (size_t)(0x4B000000u << S) + at);
+  } else {
+    // unsigned 24-bit multiply (full rate); the host keeps W_d + 3 and H_d + 2 within 2^23
+    const unsigned c = __umul24((unsigned)((int)fy + 1), (unsigned)Wc) + (unsigned)((int)fx + 1);
+    q = *reinterpret_cast<const raw *>(img + 2 * (size_t)c);
+  }
   float p00, p01, p10, p11;
   if constexpr (sizeof(TS) == 4) {
-    const float4 a = reinterpret_cast<const float4 *>(img)[c];
-    p00 = a.x; p01 = a.y; p10 = a.z; p11 = a.w;
+    p00 = q.x; p10 = q.y; p01 = q.z; p11 = q.w;
   } else {
-    const uint2 a = reinterpret_cast<const uint2 *>(img)[c];
-    unpack2(a.x, TS{}, p00, p01);
-    unpack2(a.y, TS{}, p10, p11);
+    unpack2(q.x, TS{}, p00, p10);
+    unpack2(q.y, TS{}, p01, p11);
   }
   const float p0 = lerp_ref(p00, p01, xd);
   const float p1 = lerp_ref(p10, p11, xd);
@@ -918,7 +941,7 @@ __device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, 
 // :84-118 (kernel); texture variant cone_backprojector_3D_CudaKernel_hardware_interp.cu.cc:55-87.
 // =====================================================================================
 struct BpProblem {
-  const void *cells;     // detector cells, [n][(H_d + 2) (W_d + 2)] x 4
+  const void *cells;     // detector cells, [n][(H_d + 2) (W_d + 3)] x 2
   float *vol;            // [D][H][W]
   const float *P;        // [n][12]
   const float *mult;     // [1]
@@ -983,9 +1006,9 @@ __device__ __forceinline__ void bp_block(const BpProblem &Q, int tx, int ty, int
     // accumulation would hold here in one pass, so chunked calls reproduce it exactly
     acc[q] = ((Q.flags & kBpContinue) && k0 + q < z1) ? Q.vol[((size_t)(k0 + q) * H + j) * W + i] : 0.0f;
   }
-  const int Wc = Wd + 2;
-  const size_t img_stride = (size_t)(Hd + 2) * Wc * 4;
-  const TS *img = static_cast<const TS *>(Q.cells) + (FIDX ? (size_t)(Wc + 1) * 4 : 0);
+  const int Wc = det_cols(Wd);
+  const size_t img_stride = det_image(Hd, Wd) * 2;
+  const TS *img = static_cast<const TS *>(Q.cells);
   const float *Pm = Q.P;
   const float fW = (float)Wd, fH = (float)Hd;
 
@@ -1123,9 +1146,11 @@ template <typename TS> static bool fwd_byte_offsets(int D, int H, int W) {
   const long long plane = (long long)(H + CellLayout<TS>::kYExtra) * (D + CellLayout<TS>::kZExtra);
   return W + 2 < (1 << 23) && 8 * plane < (1LL << 23) && 8 * (W + 2) * plane <= 0xB5000000LL;
 }
+// Cells the backprojection's workspace is sized for, four elements each; the two-element cells
+// fill about half of it.
 static size_t det_cells(int n, int Hd, int Wd) { return (size_t)n * (Hd + 2) * (Wd + 2); }
-// Whether the backprojection may form detector cell offsets with one float FMA (exact below 2^24).
-static bool det_fidx(int Hd, int Wd) { return (long long)(Hd + 2) * (Wd + 2) <= (1LL << 24); }
+// Whether the backprojection may form its cell offsets in floats (sample_det).
+static bool det_fidx(int Hd, int Wd) { return (long long)(Hd + 2) * det_cols(Wd) < (1LL << 23); }
 
 // A dispatch's grid size is a 32-bit count of work-items, so a 1-D grid of 256-lane blocks
 // holds at most 2^24 - 1 blocks; grid y and z hold at most 65535 blocks here.
@@ -1217,7 +1242,7 @@ static void launch_det_cells(const void *sino, void *cells, int images, int Hd, 
                              hipStream_t stream) {
   const int Hc = Hd + 2;
   const int runs = (Hc + kDetCellRows - 1) / kDetCellRows;
-  const dim3 grid((unsigned)((Wd + 2 + 255) / 256), (unsigned)(runs < kMaxGridYZ ? runs : kMaxGridYZ),
+  const dim3 grid((unsigned)((det_cols(Wd) + 255) / 256), (unsigned)(runs < kMaxGridYZ ? runs : kMaxGridYZ),
                   (unsigned)(images < kMaxGridYZ ? images : kMaxGridYZ));
   build_det_cells_kernel<TS><<<grid, dim3(256), 0, stream>>>((const TS *)sino, (TS *)cells, Hd, Wd,
                                                              images);
@@ -1240,7 +1265,7 @@ static void launch_bp(bool hw, const void *cells, float *vol, const float *P, co
   // grid z = batch items x z blocks, at most 65535 per launch: split the z blocks; grid x =
   // the items of a z block, at most kMaxGridX (rounded down to a multiple of 8) per launch
   const int per = kMaxGridYZ / B;
-  const size_t cs = det_cells(n, Hd, Wd) * 4;
+  const size_t cs = det_image(Hd, Wd) * 2 * n;
   const int items = bp_items_per_z((W + 15) / 16, (H + 15) / 16);
   const int max_x = (int)(kMaxGridX / kXcds * kXcds);
   for (int zb0 = 0; zb0 < zblocks; zb0 += per) {
