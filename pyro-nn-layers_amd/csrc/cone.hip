@@ -893,14 +893,15 @@ __global__ void build_det_cells_kernel(const TS *__restrict__ sino, TS *__restri
 }
 
 // Bilinear sample, lerp x then y (cone_backprojector_3D_CudaKernel.cu.cc:55-82),
-// zero outside the detector.  img is the view's first cell, (-1, -1).
+// zero outside the detector: the load and fractions (det_fetch), the blend (det_blend).  img is
+// the view's first cell, (-1, -1).
 // FIDX: the host guarantees (H_d + 2)(W_d + 3) < 2^23, so with the bias 2^23 the cell index is an
 // exact float in [2^23, 2^24) whose bits, shifted by the cell size, are a 32-bit byte offset from
 // an address moved by the shifted exponent bits: three instructions and a load from a uniform
 // base.
 template <typename TS, bool HW, bool FIDX>
-__device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, float u, float v,
-                                            float fW, float fH) {
+__device__ __forceinline__ typename DetLoad<TS>::raw det_fetch(const TS *__restrict__ img, int Wc, float u, float v,
+                                                               float fW, float fH, float &xd, float &yd) {
   typedef typename DetLoad<TS>::raw raw;
   constexpr int S = DetLoad<TS>::kShift;
   if (HW) {  // tex2DLayered(u + 0.5, v + 0.5, n)
@@ -910,16 +911,19 @@ __device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, 
   u = clamp_apron(u, fW);
   v = clamp_apron(v, fH);
   const float fx = floorf(u), fy = floorf(v);
-  const float xd = u - fx, yd = v - fy;
-  raw q;
+  xd = u - fx;
+  yd = v - fy;
   if constexpr (FIDX) {
     const uint32_t at = __float_as_uint(fmaf(fy, (float)Wc, fx + (0x1p23f + (float)(Wc + 1)))) << S;
-    q = *reinterpret_cast<const raw *>(reinterpret_cast<const char *>(img) - (size_t)(0x4B000000u << S) + at);
+    return *reinterpret_cast<const raw *>(reinterpret_cast<const char *>(img) - (size_t)(0x4B000000u << S) + at);
   } else {
     // unsigned 24-bit multiply (full rate); the host keeps W_d + 3 and H_d + 2 within 2^23
     const unsigned c = __umul24((unsigned)((int)fy + 1), (unsigned)Wc) + (unsigned)((int)fx + 1);
-    q = *reinterpret_cast<const raw *>(img + 2 * (size_t)c);
+    return *reinterpret_cast<const raw *>(img + 2 * (size_t)c);
   }
+}
+template <typename TS>
+__device__ __forceinline__ float det_blend(typename DetLoad<TS>::raw q, float xd, float yd) {
   float p00, p01, p10, p11;
   if constexpr (sizeof(TS) == 4) {
     p00 = q.x; p10 = q.y; p01 = q.z; p11 = q.w;
@@ -930,6 +934,12 @@ __device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, 
   const float p0 = lerp_ref(p00, p01, xd);
   const float p1 = lerp_ref(p10, p11, xd);
   return lerp_ref(p0, p1, yd);
+}
+template <typename TS, bool HW, bool FIDX>
+__device__ __forceinline__ float sample_det(const TS *__restrict__ img, int Wc, float u, float v, float fW, float fH) {
+  float xd, yd;
+  const typename DetLoad<TS>::raw q = det_fetch<TS, HW, FIDX>(img, Wc, u, v, fW, fH, xd, yd);
+  return det_blend<TS>(q, xd, yd);
 }
 
 // =====================================================================================
@@ -1012,7 +1022,34 @@ __device__ __forceinline__ void bp_block(const BpProblem &Q, int tx, int ty, int
   const float *Pm = Q.P;
   const float fW = (float)Wd, fH = (float)Hd;
 
-  for (int view = 0; view < n; ++view, img += img_stride) {
+  int view = 0;
+  if constexpr (ZPT == 1) {
+    // the variant of launches with few blocks: four views at a time, their reciprocals and
+    // loads in flight together, where one view's chain would be waited for after the other
+    constexpr int U = 4;
+    for (; view + U <= n; view += U, img += U * img_stride) {
+      float w[U], f[U];
+      bool ok = true;
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const float *m = Pm + (view + k) * 12;
+        w[k] = fmaf(m[10], z[0], fmaf(m[9], y, m[8] * x)) + m[11];
+        ok = ok && rcp_fast_ok(w[k]);
+      }
+      if (!__all(ok)) break;  // the rest one by one, with the IEEE division where it is needed
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const float *m = Pm + (view + k) * 12;
+        w[k] = rcp_fast(w[k]);
+        const float uu = (fmaf(m[2], z[0], fmaf(m[1], y, m[0] * x)) + m[3]) * w[k];
+        const float vv = (fmaf(m[6], z[0], fmaf(m[5], y, m[4] * x)) + m[7]) * w[k];
+        f[k] = sample_det<TS, HW, FIDX>(img + k * img_stride, Wc, uu, vv, fW, fH);
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) acc[0] = fmaf(f[k] * w[k], w[k], acc[0]);
+    }
+  }
+  for (; view < n; ++view, img += img_stride) {
     const float *m = Pm + view * 12;
     const float tu = fmaf(m[1], y, m[0] * x);
     const float tv = fmaf(m[5], y, m[4] * x);
@@ -1028,12 +1065,19 @@ __device__ __forceinline__ void bp_block(const BpProblem &Q, int tx, int ty, int
       if (w0 != 0.0f) {
         const float ww = rcp_rn(w0);
         const float uu = (fmaf(m[2], z[0], tu) + m[3]) * ww;
+        // All loads first: left to itself, the compiler schedules some variants of this loop with
+        // each load next to its use (16-bit items kernel, 8 voxels per lane: 256^3 / 360 views
+        // 6.1 against 3.1 ms).
+        typename DetLoad<TS>::raw cell[ZPT];
+        float xd, yd[ZPT];
 #pragma unroll
         for (int q = 0; q < ZPT; ++q) {
           const float vv = (fmaf(m[6], z[q], tv) + m[7]) * ww;
-          const float f = sample_det<TS, HW, FIDX>(img, Wc, uu, vv, fW, fH);
-          acc[q] = fmaf(f * ww, ww, acc[q]);
+          cell[q] = det_fetch<TS, HW, FIDX>(img, Wc, uu, vv, fW, fH, xd, yd[q]);
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < ZPT; ++q) acc[q] = fmaf(det_blend<TS>(cell[q], xd, yd[q]) * ww, ww, acc[q]);
         continue;
       }
     }
@@ -1232,10 +1276,17 @@ static void launch_fwd_direct(bool hw, const void *vol, float *sino, const float
   }
 }
 
-// z voxels per lane: 8 for f32 and bf16 detector cells, 4 for f16 ones (measured on the
-// 512^3 / 720-view / 1024x768 workload: f32 63.0 against 70.9 ms with 4, bf16 53.7 against
-// 57.7 ms, f16 56.9 ms with 4 against 125.9 ms with 8).
-template <typename TS> constexpr int bp_zpt() { return std::is_same<TS, _Float16>::value ? 4 : 8; }
+// z voxels per lane by the 256-lane blocks that 8 would give (the device holds 5 per CU, 1280):
+// 1 below one block per CU, 4 below three, 8 beyond.  With few blocks a block's time is its
+// chain of views, which fewer voxels per lane shorten (1, with four views in flight, most); with
+// many, one reciprocal and one column for 8 voxels count.  Measured per volume (f32, 8 / 4 / 1
+// voxels): 24^3, 12 blocks, 55 / 47 / 21 us; 64^3, 128 blocks, 125 / 101 / 56; 80^3, 250, 129 /
+// 104 / 95; 77 x 101 x 90, 420, 102 / 84 / 97; 110^3, 686, 142 / 130 / 183; 128^3, 1024, 246 /
+// 265 / 388; 512^3 53.2 / 57.5 / 95.9 ms (bf16 50.5 / 53.0, f16 50.0 / 51.9).
+static int bp_zpt(int nz, int H, int W, int B) {
+  const long long blocks = (long long)((nz + 7) / 8) * ((H + 15) / 16) * ((W + 15) / 16) * B;
+  return blocks < 256 ? 1 : blocks < 768 ? 4 : 8;
+}
 
 template <typename TS>
 static void launch_det_cells(const void *sino, void *cells, int images, int Hd, int Wd,
@@ -1254,13 +1305,10 @@ static bool bp_plane_fits(int H, int W) {
   return (long long)((W + 15) / 16) * ((H + 15) / 16) < (long long)INT32_MAX - kXcds;
 }
 
-template <typename TS>
-static void launch_bp(bool hw, const void *cells, float *vol, const float *P, const float *mult,
-                      const float *spacing, const float *origin, int B, int D, int H, int W, int n,
-                      int Hd, int Wd, hipStream_t stream, int flags = kBpScale, int z0 = 0,
-                      int z1 = -1) {
-  constexpr int Z = bp_zpt<TS>();
-  if (z1 < 0) z1 = D;
+template <typename TS, int Z>
+static void launch_bp_z(bool hw, const void *cells, float *vol, const float *P, const float *mult,
+                        const float *spacing, const float *origin, int B, int D, int H, int W, int n,
+                        int Hd, int Wd, hipStream_t stream, int flags, int z0, int z1) {
   const int zblocks = (z1 - z0 + Z - 1) / Z;
   // grid z = batch items x z blocks, at most 65535 per launch: split the z blocks; grid x =
   // the items of a z block, at most kMaxGridX (rounded down to a multiple of 8) per launch
@@ -1287,6 +1335,17 @@ static void launch_bp(bool hw, const void *cells, float *vol, const float *P, co
       }
     }
   }
+}
+
+template <typename TS>
+static void launch_bp(bool hw, const void *cells, float *vol, const float *P, const float *mult,
+                      const float *spacing, const float *origin, int B, int D, int H, int W, int n,
+                      int Hd, int Wd, hipStream_t stream, int flags = kBpScale, int z0 = 0,
+                      int z1 = -1) {
+  if (z1 < 0) z1 = D;
+  const int zpt = bp_zpt(z1 - z0, H, W, B);
+  const auto launch = zpt == 8 ? launch_bp_z<TS, 8> : zpt == 4 ? launch_bp_z<TS, 4> : launch_bp_z<TS, 1>;
+  launch(hw, cells, vol, P, mult, spacing, origin, B, D, H, W, n, Hd, Wd, stream, flags, z0, z1);
 }
 
 }  // namespace pyronn
@@ -1828,7 +1887,7 @@ extern "C" int pyronn_cone_backprojection3d_batched(const pyronn_cone_problem *p
   PYRONN_CHECK_ARG(((uintptr_t)workspace & 15) == 0, "cone_backprojection3d_batched: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const bool hw = hardware_interp != 0;
-  const int z = z_per_lane > 0 ? z_per_lane : (dtype == PYRONN_F16 ? 4 : 8);
+  const int z = z_per_lane > 0 ? z_per_lane : 8;
   char *ws = (char *)workspace;
   if (dtype == PYRONN_F32)
     rc = z == 8 ? bp_batched<float, 8>(problems, count, hw, blocks_per_cu, ws, s)

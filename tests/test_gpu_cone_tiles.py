@@ -1,6 +1,6 @@
 """How the cone kernels deal their tiles to the XCDs, at tile counts around the 8 XCDs and the
-four strips, and the f32 forward's cell indexes at the limit of its 32-bit byte offsets, all
-against the oracle."""
+four strips, the backprojection's voxels per lane, and the f32 forward's cell indexes at the
+limit of its 32-bit byte offsets, all against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -31,6 +31,27 @@ def test_backprojection_tiles_one_to_forty(plane, storage):
     og = geo.centred_origin(shape, sp).astype(np.float32)
     P = geo.circular_projection_matrices(6, 300.0, 480.0, det, (1.5, 6.0)).astype(np.float32)
     s = np.random.default_rng(plane[0]).normal(size=(6,) + det).astype(np.float32)
+    s = torch.tensor(s).to(gh.DT[storage][1]).float().numpy()
+    got = gh.cone_backward(s, P, sp, og, shape, storage=storage)[0]
+    ref, _ = orc.cone_backward(s, P, shape, sp, og)
+    assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("tilt", [0.0, 1e-4])
+@pytest.mark.parametrize("storage", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape, n", [
+    ((13, 30, 20), 3),       # 8 blocks of 8 voxels per lane: one voxel per lane, fewer views than four at a time
+    ((80, 77, 75), 9),       # 250 blocks: one voxel per lane, two groups of views and one more
+    ((61, 120, 131), 5),     # 576 blocks: four voxels per lane
+    ((43, 200, 170), 5),     # 858 blocks: eight
+])
+def test_backprojection_voxels_per_lane(shape, n, storage, tilt):
+    det = (90, 150)
+    sp = np.ones(3, np.float32)
+    og = geo.centred_origin(shape, sp).astype(np.float32)
+    P = geo.circular_projection_matrices(n, 400.0, 640.0, det, (1.5, 2.2)).astype(np.float32)
+    P[:, 2, 2] += np.float32(tilt)   # depth varies along z: no column shares its reciprocal
+    s = np.random.default_rng(n).normal(size=(n,) + det).astype(np.float32)
     s = torch.tensor(s).to(gh.DT[storage][1]).float().numpy()
     got = gh.cone_backward(s, P, sp, og, shape, storage=storage)[0]
     ref, _ = orc.cone_backward(s, P, shape, sp, og)
