@@ -269,7 +269,7 @@ __device__ float march2d_group(const TS *__restrict__ img, int W, int H, float o
 // iteration cap) around loads whose latency nothing covered.  Here a sample takes 39, and a
 // wave's load 22 cycles of the texture-address unit (16 for one 128-byte line per quad):
 // that unit is 88% busy and VALU issue at 0.39 of its 0.44-0.5 per SIMD and cycle.  Parallel
-// 256^2 / 180 views x 363 / step 0.2: 32 images 4300 -> 1420 us, one 282 -> 94; fan 512^2 /
+// 256^2 / 180 views x 363 / step 0.2: 32 images 4300 -> 1390 us, one 282 -> 83; fan 512^2 /
 // 360 x 725 / step 0.5: 535 -> 158; fan 301 x 277 f16, spacing 0.7, one image: 522 -> 124.
 // A second copy with x and y exchanged, for rays along y, was no faster (1496 us, 180 us):
 // a quad's four samples span less than two pixels at these steps.
@@ -382,23 +382,37 @@ __device__ __forceinline__ float blend_pairs(TS, typename PairLoad<TS>::raw v, f
   return lerp_ref(lerp_ref(to_f32(a[0]), to_f32(b[0]), xd), lerp_ref(to_f32(a[1]), to_f32(b[1]), xd), yd);
 }
 
-// Value of lane J of this lane's group of G (all lanes of the group active): DPP quad_perm
-// for quads, row_newbcast for rows of 16.
-template <int G, int J>
-__device__ __forceinline__ float group_bcast(float f) {
-  static_assert(G == 4 || G == 16, "a quad or a row of lanes");
-  constexpr int ctrl = G == 4 ? J * 0x55 : 0x150 + J;
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), ctrl, 0xf, 0xf, true));
+// Value of lane J of this lane's quad, and of the lane N (4, 8 or 12) places on in its row of
+// 16 (DPP; all lanes of the wave are active).
+template <int J> __device__ __forceinline__ float quad_value(float f) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), J * 0x55, 0xf, 0xf, true));
 }
-template <int G, int J = 0>
-__device__ __forceinline__ float group_sum(float pix, float f) {  // pix + f(0) + f(1) + ... in lane order
-  if constexpr (J < G) return group_sum<G, J + 1>(pix + group_bcast<G, J>(f), f);
+template <int N> __device__ __forceinline__ float row_ahead(float f) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x100 + N, 0xf, 0xf, true));
+}
+// pix + f(0) + f(1) + ... over the G lanes of a group, in lane order; right in the group's
+// first quad, which is enough.
+__device__ __forceinline__ float quad_sum(float pix, float f) {
+  pix += quad_value<0>(f);
+  pix += quad_value<1>(f);
+  pix += quad_value<2>(f);
+  return pix + quad_value<3>(f);
+}
+template <int G> __device__ __forceinline__ float group_sum(float pix, float f) {
+  static_assert(G == 4 || G == 8 || G == 16, "quads of one row of lanes");
+  pix = quad_sum(pix, f);
+  if constexpr (G >= 8) pix = quad_sum(pix, row_ahead<4>(f));
+  if constexpr (G >= 16) {
+    pix = quad_sum(pix, row_ahead<8>(f));
+    pix = quad_sum(pix, row_ahead<12>(f));
+  }
   return pix;
 }
-template <int G, int J = 0>
-__device__ __forceinline__ float group_max(float m, float f) {
-  if constexpr (J < G) return group_max<G, J + 1>(fmaxf(m, group_bcast<G, J>(f)), f);
-  return m;
+// The largest f of the group, in its first quad.
+template <int G> __device__ __forceinline__ float group_max(float f) {
+  if constexpr (G >= 16) f = fmaxf(f, row_ahead<8>(f));
+  if constexpr (G >= 8) f = fmaxf(f, row_ahead<4>(f));
+  return fmaxf(fmaxf(quad_value<0>(f), quad_value<1>(f)), fmaxf(quad_value<2>(f), quad_value<3>(f)));
 }
 
 // Emits nothing; the compiler moves no load across it (it would sink the load of the next
@@ -407,21 +421,25 @@ __device__ __forceinline__ void keep_load_here() { asm volatile("" ::: "memory")
 
 // The march of march2d with the samples of one ray spread over G lanes: lane q of the group
 // takes samples q, q + G, ...  Each lane steps its own alpha by G float additions of step,
-// which are the additions of the one-lane recurrence, and every lane adds the G values of a
-// round in sample order, so all G lanes hold the one-lane sum, bit for bit; a lane past the
-// end adds -0.0, which changes no float.  The load of the next round is issued before the
-// current one is blended; positions past the end are clamped into the copy like any other.
-// The entrance sample and the tail are computed by all lanes alike.  CAP: with the reference
-// march's iteration cap (see proj2d_pairs_kernel).
+// which are the additions of the one-lane recurrence, and the lanes of the group's first quad
+// add the G values of a round in sample order: the one-lane sum, bit for bit.  A lane past the
+// end (alpha only grows, so the samples that exist are a prefix of a round) adds -0.0, which
+// changes no float.  Quads stop by themselves, by their first lane's alpha (their loads then
+// cost the address path next to nothing: 638 against 656 us for a step of 6 fan images), larger
+// groups with the wave's last ray.  The load of the next round is
+// issued before the current one is blended; positions past the end are clamped into the copy
+// like any other.  The entrance sample and the tail are computed by all lanes alike.  CAP: with
+// the reference march's iteration cap (see proj2d_pairs_kernel).  The result is right in the
+// group's first quad.
 template <typename TS, int DIV, bool CAP, int G>
 __device__ __forceinline__ float march2d_pairs(const PairImage &im, const Ray2d &r, float amin, float amax,
                                                float step, int q) {
   typedef typename PairLoad<TS>::raw raw;
-  if (!(amin < amax)) return 0.0f;
+  const bool any = amin < amax;
   const int cap = CAP ? march_cap(amin, amax, step) : 0;
   float xa, ya, xb, yb;
   raw va = fetch2d<TS, DIV>(im, r, amin, xa, ya), vb;
-  float pix = fmaf(0.5f, blend_pairs(TS{}, va, xa, ya), 0.0f);
+  float pix = any ? fmaf(0.5f, blend_pairs(TS{}, va, xa, ya), 0.0f) : 0.0f;
   float last = amin;  // alpha of this lane's last sample so far
   float a = amin + step;
 #pragma unroll
@@ -429,31 +447,34 @@ __device__ __forceinline__ float march2d_pairs(const PairImage &im, const Ray2d 
     const float nx = a + step;
     a = q >= j ? nx : a;
   }
-  int it = 0;
+  int it = q;
   va = fetch2d<TS, DIV>(im, r, a, xa, ya);
-  // Two rounds per pass, so that no cell moves between registers.  The first lane's alpha
-  // decides for the group: alpha only grows, so the samples that exist are a prefix of a round.
-  while (group_bcast<G, 0>(a) < amax && (!CAP || it < cap)) {
+  // two rounds per pass, so that no cell moves between registers
+  const auto more = [&] {
+    if constexpr (G == 4) return quad_value<0>(a) < amax && (!CAP || it - q < cap);
+    return (bool)__any(a < amax && (!CAP || it < cap));
+  };
+  while (more()) {
     float an = a;
 #pragma unroll
     for (int j = 0; j < G; ++j) an += step;
     vb = fetch2d<TS, DIV>(im, r, an, xb, yb);
-    const bool oka = a < amax && (!CAP || it + q < cap);
+    const bool oka = a < amax && (!CAP || it < cap);
     last = oka ? a : last;
     pix = group_sum<G>(pix, oka ? blend_pairs(TS{}, va, xa, ya) : -0.0f);
     a = an;
 #pragma unroll
     for (int j = 0; j < G; ++j) a += step;
     va = fetch2d<TS, DIV>(im, r, a, xa, ya);
-    const bool okb = an < amax && (!CAP || it + G + q < cap);
+    const bool okb = an < amax && (!CAP || it + G < cap);
     last = okb ? an : last;
     pix = group_sum<G>(pix, okb ? blend_pairs(TS{}, vb, xb, yb) : -0.0f);
     it += 2 * G;
     keep_load_here();
   }
   pix *= step;
-  if (pix > 0.0f) {
-    const float alast = group_max<G>(last, last);
+  const float alast = group_max<G>(last);
+  if (any && pix > 0.0f) {
     va = fetch2d<TS, DIV>(im, r, alast, xa, ya);
     vb = fetch2d<TS, DIV>(im, r, amax, xb, yb);
     const float flast = blend_pairs(TS{}, va, xa, ya);
@@ -868,11 +889,13 @@ static void launch_proj2d_g(dim3 grid, const void *volume, int dtype, int H, int
         (const _Float16 *)volume, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det, step_factor);
 }
 
-// Rays per launch below which a ray gets 16 lanes instead of 4: with 4 the launch would have
-// less than two waves per SIMD, each waiting for its own latencies (64^2 / 60 views x 95, 5700
-// rays: 11 against 18 us; 16650 rays: 25 against 31; 65340 rays: 119 against 94 the other way,
-// the 16 broadcasts of a round costing more than the latency they hide).
-constexpr long long kRowRayLimit = 32768;
+// Rays per launch below which a ray gets 16 or 8 lanes instead of 4: a wave of a launch with few
+// rays issues an instruction every 8 cycles or so however independent they are, so a long ray's
+// time is its own instruction count; more lanes shorten it, at more additions per sample.
+// Measured with 4 / 8 / 16 lanes (us; parallel images, step 0.2): 2400 rays 12.7 / 9.6 / 8.4, 11400
+// 17.5 / 13.4 / 12.7, 12600 25.8 / 18.5 / 20.0, 38250 54.1 / 48.9 / 66.1, 65340 91.4 / 83.0 / 124.7,
+// 130680 137 / 142 / 211, 2.1 million 1388 / 1689 / 2912.
+constexpr long long kRowRays = 12000, kHalfRowRays = 65536;
 
 template <typename TS, bool FAN>
 static void launch_pairs(const void *volume, int batch, int H, int W, const float *vo, const float *dor,
@@ -881,17 +904,16 @@ static void launch_pairs(const void *volume, int batch, int H, int W, const floa
   TS *pairs = (TS *)ws;
   build_pairs_kernel<TS><<<dim3((unsigned)((pair_cols(W) + 255) / 256), (unsigned)pair_rows(H), (unsigned)batch),
                            dim3(256), 0, s>>>((const TS *)volume, pairs, H, W);
-  const int G = (long long)det * n * batch < kRowRayLimit ? 16 : 4;
+  const long long nrays = (long long)det * n * batch;
+  const int G = nrays < kRowRays ? 16 : nrays < kHalfRowRays ? 8 : 4;
   // one wave per block: the rays of a view differ in length, and the dispatch evens out
   // single waves best (256-lane blocks: 2168 against 1922 us for 16 fan 512^2 images, 171
   // against 158 us for one; a batch of 32 parallel 256^2 images is the same)
   const dim3 grid((unsigned)(((long long)G * det + 63) / 64), n, batch);
-  if (G == 16)
-    proj2d_pairs_kernel<TS, FAN, 16><<<grid, dim3(64), 0, s>>>(pairs, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n,
-                                                               det, step_factor);
-  else
-    proj2d_pairs_kernel<TS, FAN, 4><<<grid, dim3(64), 0, s>>>(pairs, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n,
-                                                              det, step_factor);
+  const auto kernel = G == 16  ? proj2d_pairs_kernel<TS, FAN, 16>
+                      : G == 8 ? proj2d_pairs_kernel<TS, FAN, 8>
+                               : proj2d_pairs_kernel<TS, FAN, 4>;
+  kernel<<<grid, dim3(64), 0, s>>>(pairs, sino, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det, step_factor);
 }
 
 template <bool FAN>

@@ -42,7 +42,8 @@ def _run(fan, img, sp, n, det, ds, step, sid, storage=torch.float32, arc=2 * mat
     (3, 70, (0.5, 0.5), 9, 65),          # power-of-two spacing below the box's 0.5 mm edge
     (70, 3, (0.7, 1.3), 9, 66),          # refined division, two spacings
     (33, 31, (0.3, 0.3), 7, 61),         # coordinates below -1: the copy's second border cell
-    (40, 44, (0.9, 1.0), 300, 110),      # 33000 rays: 4 lanes per ray, det no multiple of 16
+    (40, 44, (0.9, 1.0), 300, 110),      # 33000 rays: 8 lanes per ray, det no multiple of 8
+    (21, 26, (0.8, 0.8), 550, 121),      # 66550 rays: 4 lanes per ray, det no multiple of 16
     (24, 24, (1e-19, 1e-19), 3, 17),     # a spacing the refined division does not serve
 ])
 def test_pairs_match_the_oracle(fan, storage, H, W, sp, n, det):
