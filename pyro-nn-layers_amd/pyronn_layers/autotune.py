@@ -9,8 +9,8 @@ Tunable parameters (all preserve results bit for bit):
                    (0: one workgroup per item; otherwise a persistent grid)
 Each candidate is timed with HIP events (best of `reps` after one warm-up) and
 the winner is cached in a JSON file keyed by the batch signature (shapes,
-views, detector sizes, storage dtype, interpolation mode, device name), so a later
-call with the same signature reuses it without timing.
+views, detector sizes, storage dtype, interpolation mode, device name) and the kernels'
+generation, so a later call with the same signature reuses it without timing.
 """
 from __future__ import annotations
 
@@ -25,6 +25,9 @@ from . import geometry as geo
 
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "pyronn_mi_autotune.json")
 
+# Part of the cache key: raised whenever kernels change enough to move the winners (a 32x8 tile
+# kept from the kernels before would cost 10% in the batched forward).
+KERNELS = 2
 
 TILE_SHAPES = {0: "16x16/4x16", 1: "8x32/2x32", 2: "32x8/8x8", 3: "16x16/8x8"}   # tile / wave (cols x rows)
 
@@ -33,7 +36,7 @@ def signature(kind: str, tensors: Sequence[torch.Tensor], geometries: Sequence[g
               hardware_interp: bool = False) -> str:
     dev = torch.cuda.get_device_name(tensors[0].device)
     parts = [f"{tuple(g.volume_shape)}:{g.n_views}:{tuple(g.detector_shape)}" for g in geometries]
-    return f"{kind}|{tensors[0].dtype}|hw={int(bool(hardware_interp))}|{dev}|" + ";".join(parts)
+    return f"{kind}|k{KERNELS}|{tensors[0].dtype}|hw={int(bool(hardware_interp))}|{dev}|" + ";".join(parts)
 
 
 def _time(fn, reps: int) -> float:
