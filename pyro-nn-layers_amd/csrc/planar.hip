@@ -697,8 +697,10 @@ back2d_kernel(const TS *__restrict__ sino, float *__restrict__ vol, const float 
 // back with two broadcast reads), both quotients share one correctly rounded reciprocal
 // (div_spacing's two corrections), and rcp_sqrt_fast serves the weight: about 68 per update.
 // The parallel kernel's 15 leave it to the address path, one pair load per update.  512^2 fan,
-// 360 views x 725: 221 -> 133 us (8 images 1233 -> 805); 256^2 parallel, 180 views x 363: 45 ->
-// 23.5 us (32 images 309 -> 181).
+// 360 views x 725: 221 -> 126 us (8 images 1233 -> 829); 256^2 parallel, 180 views x 363: 45 ->
+// 23.5 us (32 images 309 -> 181).  A test per view for the rare distances that rcp_sqrt_fast does
+// not serve kept the views' chains from overlapping: 52 x 48 fan, 44 views, 25.5 us with it (24.9
+// for back2d_kernel), 14 without.
 // =====================================================================================
 __host__ __device__ inline int row_len(int det) { return det + 4; }
 
@@ -745,8 +747,13 @@ struct alignas(16) ViewTerms {
 };
 constexpr int kBackViews = 128;
 
-// The fan pixel's detector coordinate in mm and distance weight.  FAST: see back2d_rows_kernel.
-template <bool FAST>
+// The fan pixel's detector coordinate in mm and distance weight.  FAST: see back2d_rows_kernel;
+// SQRT: rcp_sqrt_ok holds for the squared distance.
+__device__ __forceinline__ float fan_distance2(const ViewTerms &v, float pcx, float pcy) {
+  const float a = pcx - v.srx, c = pcy - v.sry;
+  return fmaf(c, c, a * a);
+}
+template <bool FAST, bool SQRT>
 __device__ __forceinline__ void fan_pixel(const ViewTerms &v, float pcx, float pcy, float &s, float &dw) {
   const float a = pcx - v.srx, c = pcy - v.sry;
   const float den = fmaf(-c, v.d, a * v.b);
@@ -762,9 +769,9 @@ __device__ __forceinline__ void fan_pixel(const ViewTerms &v, float pcx, float p
     iy = ny / den;
   }
   s = fmaf(iy, v.d1, ix * v.d0);
-  if (den < 0.000001f && den > -0.000001f) s = __builtin_nanf("");  // helper_geometry_gpu.h:28-44
+  s = (den < 0.000001f && den > -0.000001f) ? __builtin_nanf("") : s;  // helper_geometry_gpu.h:28-44
   const float t = fmaf(c, c, a * a);
-  dw = (FAST && rcp_sqrt_ok(t)) ? rcp_sqrt_fast(t) : rcp_rn(sqrtf(t));
+  dw = SQRT ? rcp_sqrt_fast(t) : rcp_rn(sqrtf(t));
 }
 
 template <typename TS, bool FAN, bool FAST, int DIV, int P>
@@ -777,8 +784,10 @@ __device__ __forceinline__ void back2d_rows(const TS *__restrict__ rows, const f
   for (int v0 = 0; v0 < n; v0 += kBackViews) {
     const int nv = n - v0 < kBackViews ? n - v0 : kBackViews;
     __syncthreads();
+    bool near = true;  // no source of these views is beyond 2^42 mm (FAST bounds the distances)
     for (int k = threadIdx.x; k < nv; k += blockDim.x) {
       const float c0 = rb[(v0 + k) * 2 + 0], c1 = rb[(v0 + k) * 2 + 1];
+      near = near && fmaxf(fabsf(c0), fabsf(c1)) <= 0x1p20f;
       ViewTerms t{};
       if (FAN) {
         t.d0 = -c1;
@@ -796,19 +805,46 @@ __device__ __forceinline__ void back2d_rows(const TS *__restrict__ rows, const f
       }
       terms[k] = t;
     }
-    __syncthreads();
-#pragma unroll 4  // four views in flight: a lane's chain per view is long and its load exposed
-    for (int k = 0; k < nv; ++k, base += (size_t)row_len(det) * sizeof(TS)) {
-      if (FAN) {
+    near = __syncthreads_and(near);
+    const size_t row_bytes = (size_t)row_len(det) * sizeof(TS);
+    if constexpr (FAN) {
+      // U views at a time without a branch between them, so that their chains and loads overlap:
+      // one test for all of them that rcp_sqrt_fast serves every distance (a NaN passes and
+      // stays one)
+      constexpr int U = 4 / P;
+      int k = 0;
+      for (; FAST && near && k + U <= nv; k += U, base += U * row_bytes) {
+        float closest = 1.0f;
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+#pragma unroll
+          for (int p = 0; p < P; ++p) closest = fminf(closest, fan_distance2(terms[k + j], pcx, pcy[p]));
+        if (!__all(closest >= 0x1p-100f)) break;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          const ViewTerms t = terms[k + j];
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            float s, dw;
+            fan_pixel<true, true>(t, pcx, pcy[p], s, dw);
+            const float f = sample_row<TS>(base + j * row_bytes, fdet, div_spacing<DIV>(s - do_, ds, ids));
+            val[p] = fmaf(f * dw, dw, val[p]);
+          }
+        }
+      }
+      for (; k < nv; ++k, base += row_bytes) {
         const ViewTerms t = terms[k];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
           float s, dw;
-          fan_pixel<FAST>(t, pcx, pcy[p], s, dw);
+          fan_pixel<FAST, false>(t, pcx, pcy[p], s, dw);
           const float f = sample_row<TS>(base, fdet, div_spacing<DIV>(s - do_, ds, ids));
           val[p] = fmaf(f * dw, dw, val[p]);
         }
-      } else {
+      }
+    } else {
+#pragma unroll 4  // four views in flight: each load would be waited for alone
+      for (int k = 0; k < nv; ++k, base += row_bytes) {
         const float c0 = terms[k].srx, m1 = pcx * terms[k].sry;
 #pragma unroll
         for (int p = 0; p < P; ++p)
@@ -974,8 +1010,8 @@ static void launch_rows(const void *sino, int batch, int n, int det, const float
                           dim3(256), 0, s>>>((const TS *)sino, rows, det, nrows);
   // One pixel per lane while the blocks fit the device at once (8 of 256 lanes per CU), two
   // beyond: a few blocks past a full round run alone for as long as the round did (6 fan images
-  // of 301 x 277, 2052 blocks: 264 against 184 us; 8 of 512^2, 8192 blocks: 821 against 805),
-  // below it the second pixel only lengthens a block (512^2, 1024 blocks: 133 against 148).
+  // of 301 x 277, 2052 blocks: 264 against 184 us), below it the second pixel only lengthens a
+  // block (512^2, 1024 blocks: 133 against 148).
   const long long blocks = (long long)((W + 15) / 16) * ((H + 15) / 16) * batch;
   if (blocks <= 2048) {
     const dim3 grid((W + 15) / 16, (H + 15) / 16, batch);
