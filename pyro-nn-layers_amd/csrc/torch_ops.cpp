@@ -19,6 +19,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/Exception.h>
 #include <torch/library.h>
 
 #include <vector>
@@ -160,6 +161,17 @@ Geo2D geo2d(int64_t B, int64_t n, const at::Tensor &vo, const at::Tensor &dor, c
   return g;
 }
 
+// Workspace of the 2D operators' copies.  Undefined where there is no copy (0 bytes) and where the
+// device has no room for it: the operators then sample the data as it lies, same bits, slower.
+at::Tensor copy_workspace(size_t bytes, const at::Tensor &data) {
+  if (!bytes) return at::Tensor();
+  try {
+    return at::empty({(int64_t)bytes}, data.options().dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError &) {
+    return at::Tensor();
+  }
+}
+
 at::Tensor proj2d(bool fan, const at::Tensor &volume, at::IntArrayRef projection_shape,
                   const at::Tensor &vo, const at::Tensor &dor, const at::Tensor &vs,
                   const at::Tensor &ds, const at::Tensor *sid, const at::Tensor *sdd,
@@ -177,18 +189,17 @@ at::Tensor proj2d(bool fan, const at::Tensor &volume, at::IntArrayRef projection
   if (empty_output(out)) return out;
   // the pair copy of the images that the projection samples; none for images too large for it
   const size_t ws = pyronn_projection2d_workspace_size((int)B, (int)H, (int)W, dt);
-  at::Tensor work;
-  if (ws) work = at::empty({(int64_t)ws}, vol.options().dtype(at::kByte));
+  const at::Tensor work = copy_workspace(ws, vol);
   const float *vop = g.vo.data_ptr<float>(), *dop = g.dor.data_ptr<float>(), *vsp = g.vs.data_ptr<float>(),
               *dsp = g.ds.data_ptr<float>(), *rp = g.rays.data_ptr<float>();
   const float *sidp = fan ? g.sid.data_ptr<float>() : nullptr, *sddp = fan ? g.sdd.data_ptr<float>() : nullptr;
   float *outp = out.data_ptr<float>();
   const pyronn_stream_t st = cur_stream(vol);
   int rc;
-  if (ws && fan)
+  if (work.defined() && fan)
     rc = pyronn_fan_projection2d_ws(vol.data_ptr(), dt, (int)B, (int)H, (int)W, vop, dop, vsp, dsp, sidp, sddp, rp,
                                     (int)n, (int)det, (float)step_size, outp, work.data_ptr(), ws, st);
-  else if (ws)
+  else if (work.defined())
     rc = pyronn_parallel_projection2d_ws(vol.data_ptr(), dt, (int)B, (int)H, (int)W, vop, dop, vsp, dsp, rp, (int)n,
                                          (int)det, (float)step_size, outp, work.data_ptr(), ws, st);
   else if (fan)
@@ -218,18 +229,17 @@ at::Tensor back2d(bool fan, const at::Tensor &sinogram, at::IntArrayRef volume_s
   if (empty_output(out)) return out;
   // the bordered copy of the projections that the backprojection samples
   const size_t ws = pyronn_backprojection2d_workspace_size((int)B, (int)n, (int)det, dt);
-  at::Tensor work;
-  if (ws) work = at::empty({(int64_t)ws}, sino.options().dtype(at::kByte));
+  const at::Tensor work = copy_workspace(ws, sino);
   const float *vop = g.vo.data_ptr<float>(), *dop = g.dor.data_ptr<float>(), *vsp = g.vs.data_ptr<float>(),
               *dsp = g.ds.data_ptr<float>(), *rp = g.rays.data_ptr<float>();
   const float *sidp = fan ? g.sid.data_ptr<float>() : nullptr, *sddp = fan ? g.sdd.data_ptr<float>() : nullptr;
   float *outp = out.data_ptr<float>();
   const pyronn_stream_t st = cur_stream(sino);
   int rc;
-  if (ws && fan)
+  if (work.defined() && fan)
     rc = pyronn_fan_backprojection2d_ws(sino.data_ptr(), dt, (int)B, (int)n, (int)det, vop, dop, vsp, dsp, sidp, sddp,
                                         rp, (int)H, (int)W, outp, work.data_ptr(), ws, st);
-  else if (ws)
+  else if (work.defined())
     rc = pyronn_parallel_backprojection2d_ws(sino.data_ptr(), dt, (int)B, (int)n, (int)det, vop, dop, vsp, dsp, rp,
                                              (int)H, (int)W, outp, work.data_ptr(), ws, st);
   else if (fan)

@@ -125,3 +125,34 @@ def test_rows_source_inside_the_image_and_far_lengths():
     # lengths of 2^20 mm and more take the IEEE sequences
     got, ref = _back(True, sino, (31, 29), (1.0, 1.0), 1.0, 3.0e6, off=(1.1e6, 0.0))
     assert np.array_equal(got, ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("back", [False, True])
+def test_no_room_for_the_copy(back):
+    # 67 MB of data, copies of 136 and 69 MB, an allocator that may take 16 MB more and whose free
+    # blocks of 60 MB and more (other tests leave some) are taken first
+    import pyronn_layers as pl
+    x = torch.randn(64, 512, 512, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+    dev = lambda *a: torch.tensor(a, dtype=torch.float32, device="cuda")
+    if back:
+        geom = [dev(-7.5, -7.5), dev(-255.5), dev(1.0, 1.0), dev(1.0)]
+        rays = torch.tensor(geo.parallel_ray_vectors(512, math.pi), dtype=torch.float32, device="cuda")
+        run = lambda: pl.parallel_backprojection2d(x, [16, 16], *geom, rays)
+    else:
+        geom = [dev(-255.5, -255.5), dev(-120.0), dev(1.0, 1.0), dev(8.0)]
+        rays = torch.tensor(geo.parallel_ray_vectors(4, math.pi), dtype=torch.float32, device="cuda")
+        run = lambda: pl.parallel_projection2d(x, [4, 31], *geom, rays)
+    want = run()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (16 << 20)) / total)
+        taken = []
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            for _ in range(total // (60 << 20)):
+                taken.append(torch.empty(60 << 20, dtype=torch.uint8, device="cuda"))
+        got = run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want)
