@@ -22,6 +22,16 @@ def test_forward_tiles_one_to_forty(det, storage):
     _check_views(vol, P, sp, og, det, 0.5, False, views=range(5))
 
 
+@pytest.mark.parametrize("det", [(512, 33), (497, 16), (528, 17), (496, 20), (640, 18)])
+@pytest.mark.parametrize("storage", ["bf16", "f16"])
+def test_forward_tile_rows_around_thirty_two(det, storage):
+    # 32 and 40 tile rows (whole rows per XCD in bf16), 31 and 33 (tiles one by one)
+    shape = (20, 24, 18)
+    sp, og, P = _orbit(shape, 3, 100.0, 160.0, det, (60.0 / det[0], 60.0 / det[1]))
+    vol = _rand_volume(shape, det[0], gh.DT[storage][1])
+    _check_views(vol, P, sp, og, det, 0.5, False, views=range(3))
+
+
 @pytest.mark.parametrize("plane", [(16, 16), (1, 80), (112, 33), (40, 150), (129, 65), (64, 64)])
 @pytest.mark.parametrize("storage", ["f32", "f16"])
 def test_backprojection_tiles_one_to_forty(plane, storage):
