@@ -617,12 +617,11 @@ __device__ __forceinline__ float march_ray(const TS *__restrict__ v, IT Dc, IT H
 // same number of tiles to within one, of every kind.  (Measured against whole tile rows dealt
 // to the XCDs, which also left an XCD with up to twice the mean on detectors of few rows: f32
 // 512^3 / 720 views 350 -> 333 ms, 384^3 59.5 -> 56.4, 256^3 / 400^2 detector 28.4 -> 22.7,
-// 128^3 2.06 -> 1.72; bf16 256^3 21.8 -> 17.9.  bf16 alone keeps whole tile rows on detectors of
-// 32 or more tile rows that divide by 8 (every XCD then has the same number of tiles either way):
-// 512^3 / 48 rows 237.2 against 238.5 ms, 384^3 / 40 rows 52.1 against 53.6; at 24 rows it loses,
-// 256^3 14.8 against 13.8, and f16 loses at 48, 247.4 against 244.8.  Views outer, tiles inner took
-// 534 ms where tiles outer took 483.)  The order changes only which lane computes which ray,
-// never the arithmetic of a ray.
+// 128^3 2.06 -> 1.72; bf16 256^3 21.8 -> 17.9.  With 32 or more tile rows that divide by 8, where whole
+// rows load the XCDs evenly too: bf16 512^3 / 48 rows equal, 247.7 -> 247.1, 600^3 / 56 rows 139.0 ->
+// 134.9, 300^3 / a 512 x 200 detector 9.6 -> 7.1; f16 512^3 / 200 views 99.4 -> 95.9, f32 124.6 -> 117.4.
+// Views outer, tiles inner took 534 ms where tiles outer took 483.)  The order changes only which lane
+// computes which ray, never the arithmetic of a ray.
 // Ray setup: cone_projector_3D_CudaKernel.cu.cc:197-221; march: :87-181
 // (hardware_interp: cone_projector_3D_CudaKernel_hardware_interp.cu.cc:43-142).
 // =====================================================================================
@@ -659,17 +658,9 @@ __device__ __forceinline__ void fwd_block(const FwdProblem &P, long long q) {
   const long long qq = q / kXcds;  // view fastest, then the XCD's tiles
   const long long k = qq / P.n;
   const int view = (int)(qq - k * P.n);
-  int ty, tx;
-  if (std::is_same<TS, bf16s>::value && P.tiles_y % kXcds == 0 && P.tiles_y >= 32) {
-    const int band = (int)(k / P.tiles_x);
-    ty = band * kXcds + xcd;
-    tx = (int)(k - (long long)band * P.tiles_x);
-  } else {
-    const long long t = k * kXcds + xcd;
-    if (t >= (long long)P.tiles_x * P.tiles_y) return;
-    ty = (int)(t / P.tiles_x);
-    tx = (int)(t - (long long)ty * P.tiles_x);
-  }
+  const long long t = k * kXcds + xcd;
+  if (t >= (long long)P.tiles_x * P.tiles_y) return;
+  const int ty = (int)(t / P.tiles_x), tx = (int)(t - (long long)ty * P.tiles_x);
   const int W = P.W, H = P.H, D = P.D, Hd = P.Hd, Wd = P.Wd;
   // Lanes past the detector's last column or row: in the 16-bit streamed march they march a
   // copy of the edge pixel's ray and store nothing, so that every lane of the wave takes

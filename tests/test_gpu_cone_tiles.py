@@ -25,7 +25,7 @@ def test_forward_tiles_one_to_forty(det, storage):
 @pytest.mark.parametrize("det", [(512, 33), (497, 16), (528, 17), (496, 20), (640, 18)])
 @pytest.mark.parametrize("storage", ["bf16", "f16"])
 def test_forward_tile_rows_around_thirty_two(det, storage):
-    # 32 and 40 tile rows (whole rows per XCD in bf16), 31 and 33 (tiles one by one)
+    # 31, 32, 33 and 40 tile rows of one to three tiles: rows that fill the XCDs evenly and rows that do not
     shape = (20, 24, 18)
     sp, og, P = _orbit(shape, 3, 100.0, 160.0, det, (60.0 / det[0], 60.0 / det[1]))
     vol = _rand_volume(shape, det[0], gh.DT[storage][1])
