@@ -304,7 +304,9 @@ int pyronn_cone_projection3d_batched(const pyronn_cone_problem *problems, int co
 
 size_t pyronn_cone_backprojection3d_batched_workspace_size(const pyronn_cone_problem *problems,
                                                            int count, int dtype);
-/* z_per_lane: voxels along z per lane, 4 or 8 (<= 0: 8).
+/* z_per_lane: voxels along z per lane, 4 or 8 (<= 0: 4 where 8 would
+ * give 768 workgroups or fewer, or a twentieth more voxels than 4 once the depths are rounded up to
+ * whole lanes, else 8).
  * blocks_per_cu > 0: a persistent grid of that many workgroups per CU claiming items from
  * per-XCD counters; <= 0 (default): one workgroup per item in item order (the persistent
  * grid of 8 per CU when the items exceed one dispatch's 2^24 - 1 workgroups).  Both give the

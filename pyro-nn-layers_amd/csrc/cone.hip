@@ -1278,16 +1278,47 @@ static void launch_fwd_direct(bool hw, const void *vol, float *sino, const float
   }
 }
 
+// Voxels of z ranges rounded up to whole lanes of 8 and of 4 voxels, summed over problems.  Where 8
+// per lane compute a twentieth more voxels than 4 (ranges of 1-4, 9-12, 17-20, ... up to 76-80
+// slices), the padding costs what 4 per lane lose otherwise.  Measured at 512^2 x nz, 180 views (us,
+// 8 / 4 voxels): f16 nz = 4 199 / 131, 8 203 / 211, 12 368 / 297, 20 532 / 464, 52 1198 / 1137, 68
+// 1531 / 1483, 100 2237 / 2220; f32 186 / 139, 186 / 204, 358 / 302, 533 / 466, 1242 / 1188, 1597 /
+// 1570, 2393 / 2364; bf16 as f16; with depth varying along z (no shared reciprocal) nz = 4 f16 322 / 172.
+struct BpPadding {
+  double by8 = 0, by4 = 0;
+  void add(int nz, double weight) {
+    by8 += 8 * ((nz + 7ll) / 8) * weight;
+    by4 += 4 * ((nz + 3ll) / 4) * weight;
+  }
+  bool prefers4() const { return by8 * 20 >= by4 * 21; }
+};
+
 // z voxels per lane by the 256-lane blocks that 8 would give (the device holds 5 per CU, 1280):
-// 1 below one block per CU, 4 below three, 8 beyond.  With few blocks a block's time is its
-// chain of views, which fewer voxels per lane shorten (1, with four views in flight, most); with
-// many, one reciprocal and one column for 8 voxels count.  Measured per volume (f32, 8 / 4 / 1
+// 1 below one block per CU, 4 up to three and for ranges that 8 would pad, 8 beyond.  With few blocks a
+// block's time is its chain of views, which fewer voxels per lane shorten (1, with four views in flight,
+// most); with many, one reciprocal and one column for 8 voxels count.  Measured per volume (f32, 8 / 4 / 1
 // voxels): 24^3, 12 blocks, 55 / 47 / 21 us; 64^3, 128 blocks, 125 / 101 / 56; 80^3, 250, 129 /
-// 104 / 95; 77 x 101 x 90, 420, 102 / 84 / 97; 110^3, 686, 142 / 130 / 183; 128^3, 1024, 246 /
-// 265 / 388; 512^3 53.2 / 57.5 / 95.9 ms (bf16 50.5 / 53.0, f16 50.0 / 51.9).
+// 104 / 95; 77 x 101 x 90, 420, 102 / 84 / 97; 110^3, 686, 142 / 130 / 183; 64 of 24^3, 768, 141 / 127;
+// 128^3, 1024, 246 / 265 / 388; 512^3 53.2 / 57.5 / 95.9 ms (bf16 50.5 / 53.0, f16 50.0 / 51.9).
+static long long bp_blocks8(int nz, int H, int W) {
+  return (nz + 7ll) / 8 * ((H + 15) / 16) * ((W + 15) / 16);
+}
 static int bp_zpt(int nz, int H, int W, int B) {
-  const long long blocks = (long long)((nz + 7) / 8) * ((H + 15) / 16) * ((W + 15) / 16) * B;
-  return blocks < 256 ? 1 : blocks < 768 ? 4 : 8;
+  const long long blocks = bp_blocks8(nz, H, W) * B;
+  BpPadding pad;
+  pad.add(nz, 1);
+  return blocks < 256 ? 1 : blocks <= 768 || pad.prefers4() ? 4 : 8;
+}
+// The default of a batched launch, whose kernels take 4 or 8: one choice for all its problems, by the
+// same lines (f16, 8 / 4 voxels: one problem of 40 x 60 x 50, 60 views, 82 / 60 us).
+static int bp_batched_zpt(const pyronn_cone_problem *pr, int count) {
+  long long blocks = 0;
+  BpPadding pad;
+  for (int k = 0; k < count; ++k) {
+    blocks += bp_blocks8(pr[k].D, pr[k].H, pr[k].W);
+    pad.add(pr[k].D, (double)pr[k].n_views * pr[k].H * pr[k].W);
+  }
+  return blocks <= 768 || pad.prefers4() ? 4 : 8;
 }
 
 template <typename TS>
@@ -1889,7 +1920,7 @@ extern "C" int pyronn_cone_backprojection3d_batched(const pyronn_cone_problem *p
   PYRONN_CHECK_ARG(((uintptr_t)workspace & 15) == 0, "cone_backprojection3d_batched: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const bool hw = hardware_interp != 0;
-  const int z = z_per_lane > 0 ? z_per_lane : 8;
+  const int z = z_per_lane > 0 ? z_per_lane : bp_batched_zpt(problems, count);
   char *ws = (char *)workspace;
   if (dtype == PYRONN_F32)
     rc = z == 8 ? bp_batched<float, 8>(problems, count, hw, blocks_per_cu, ws, s)

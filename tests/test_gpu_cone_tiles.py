@@ -7,6 +7,7 @@ import torch
 
 import gpu_helpers as gh
 import oracle as orc
+from pyronn_layers import batched
 from pyronn_layers import geometry as geo
 from test_gpu_limits import _check_views, _orbit, _rand_volume
 
@@ -53,7 +54,12 @@ def test_backprojection_tiles_one_to_forty(plane, storage):
     ((13, 30, 20), 3),       # 8 blocks of 8 voxels per lane: one voxel per lane, fewer views than four at a time
     ((80, 77, 75), 9),       # 250 blocks: one voxel per lane, two groups of views and one more
     ((61, 120, 131), 5),     # 576 blocks: four voxels per lane
-    ((43, 200, 170), 5),     # 858 blocks: eight
+    ((43, 200, 170), 5),     # 858 blocks of 8, a tenth of them padding: four
+    ((47, 200, 170), 5),     # 858 blocks: eight
+    ((5, 520, 410), 3),      # one slab of 8 for five slices: eight (four per lane pad as much)
+    ((4, 520, 410), 3),      # and for four: four
+    ((76, 160, 170), 2),     # the deepest range that four serve for its padding
+    ((84, 160, 170), 2),     # the first beyond
 ])
 def test_backprojection_voxels_per_lane(shape, n, storage, tilt):
     det = (90, 150)
@@ -66,6 +72,24 @@ def test_backprojection_voxels_per_lane(shape, n, storage, tilt):
     got = gh.cone_backward(s, P, sp, og, shape, storage=storage)[0]
     ref, _ = orc.cone_backward(s, P, shape, sp, og)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("shapes", [
+    ((3, 36, 40), (12, 45, 40)),        # few blocks: four voxels per lane by default
+    ((5, 300, 320), (16, 250, 340)),    # 380 + 704 blocks and no padding that four would save: eight
+    ((4, 500, 400), (12, 300, 310)),    # 800 + 760 blocks, padded: four
+])
+def test_batched_backprojection_default_voxels_per_lane(shapes, storage):
+    det, n = (20, 60), 3
+    geoms = [geo.ConeGeometry(s, (1.0, 1.0, 1.0), det, (1.5, 12.0), n, 600.0, 960.0) for s in shapes]
+    rng = np.random.default_rng(len(shapes))
+    sinos = [torch.tensor(rng.normal(size=(n,) + det)).to("cuda", gh.DT[storage][1]) for _ in shapes]
+    for x, g, got in zip(sinos, geoms, batched.cone_backprojection3d_batched(sinos, geoms)):
+        ref, _ = orc.cone_backward(x.float().cpu().numpy(), g.projection_matrices().astype(np.float32),
+                                   g.volume_shape, np.asarray(g.volume_spacing, np.float32),
+                                   np.asarray(g.volume_origin, np.float32), mult=np.float32(g.projection_multiplier))
+        assert np.array_equal(got.cpu().numpy(), ref)
 
 
 @pytest.mark.parametrize("shape, fits", [
