@@ -607,14 +607,14 @@ __device__ __forceinline__ float march_ray(const TS *__restrict__ v, IT Dc, IT H
 // (z-neighbours in one z-fastest cell column, mostly one line) rather than four columns
 // (up to four different cell columns).
 // Work order: workgroups are dispatched round-robin over the 8 XCDs, so block id
-// b runs on XCD b % 8.  The detector tiles, row by row, are dealt to the XCDs in turn, and
-// an XCD walks its tiles (outer) and views (inner).  The blocks resident on one XCD at any
-// time are therefore one or two 16 x 16 tiles over a few hundred consecutive views: the rays
-// of one pixel in consecutive views are half a degree apart, so lines fetched for one view
-// are read again by the next while they are still in that XCD's L2; all XCDs work on
-// neighbouring tiles of one row, whose rays cross the same z slab of the volume, so what one
-// XCD fetches from memory the others find in the cache behind the L2s; and every XCD has the
-// same number of tiles to within one, of every kind.  (Measured against whole tile rows dealt
+// b runs on XCD b % 8.  The detector tiles, row by row, are dealt to the XCDs in turn
+// (fwd_tile), and an XCD walks its tiles (outer) and views (inner).  The blocks resident on
+// one XCD at any time are therefore one or two 16 x 16 tiles over a few hundred consecutive
+// views: the rays of one pixel in consecutive views are half a degree apart, so lines fetched
+// for one view are read again by the next while they are still in that XCD's L2; all XCDs
+// work on neighbouring tiles of one row, whose rays cross the same z slab of the volume, so
+// what one XCD fetches from memory the others find in the cache behind the L2s; and every XCD
+// has the same number of tiles to within one.  (Measured against whole tile rows dealt
 // to the XCDs, which also left an XCD with up to twice the mean on detectors of few rows: f32
 // 512^3 / 720 views 350 -> 333 ms, 384^3 59.5 -> 56.4, 256^3 / 400^2 detector 28.4 -> 22.7,
 // 128^3 2.06 -> 1.72; bf16 256^3 21.8 -> 17.9.  With 32 or more tile rows that divide by 8, where whole
@@ -635,6 +635,7 @@ struct FwdProblem {
   const float *spacing;  // [3] (z, y, x)
   int W, H, D, n, Hd, Wd, tiles_x, tiles_y;
   long long begin;       // first work item of the problem in a batched launch (multiple of 8)
+  bool neighbours;       // order of the tiles (fwd_tile)
 };
 
 // Forward block shapes: a 256-lane block covers TC detector columns x TR rows and each of
@@ -650,17 +651,48 @@ constexpr int kFwdTiles = 4;  // 0: 16 x 16 (4 x 16 waves), 1: 8 x 32 (2 x 32), 
 __host__ __device__ constexpr int fwd_tile_cols(int t) { return t == 1 ? 8 : t == 2 ? 32 : 16; }
 __host__ __device__ constexpr int fwd_tile_rows(int t) { return t == 1 ? 32 : t == 2 ? 8 : 16; }
 
+// Tile (row by row) of XCD xcd's turn k and a view; -1: none.  The k-th eight tiles are one turn of the
+// XCDs, and each takes another of the eight in every eighth of the views: with one tile for all views an
+// XCD could have only tiles of the longest or the shortest rays, worst with 8 or 16 tile columns, where
+// it would keep its columns in every row.  Eight views at least stay together, which share what they
+// fetch (192^3, 6 views, f32 238 us undivided, 248 in twos and fours).  Measured without / with (180
+// views): 64^3, 128^2 detector, f32 345 / 290 us, bf16 281 / 248, f16 301 / 260; 128^3, 256^2 f32 2183 /
+// 2057, f16 1885 / 1723; 32^3, 64^2 f32 57.6 / 53.0; 32 volumes of 24^3, 20 views, 91 / 77; 256^3 and 512^3
+// equal.  neighbours: an XCD takes one range of adjacent tiles instead (fwd_neighbours).
+__device__ __forceinline__ int fwd_tile(int k, int xcd, int view, int n, int tiles, bool neighbours) {
+  if (neighbours) {
+    const int t0 = xcd * tiles / kXcds, t1 = (xcd + 1) * tiles / kXcds;
+    return k < t1 - t0 ? t0 + k : -1;
+  }
+  const int part = n > 8 * kXcds ? (n + kXcds - 1) / kXcds : 8;
+  const int t = k * kXcds + (xcd + view / part) % kXcds;
+  return t < tiles ? t : -1;
+}
+
+// Whether a launch of all `blocks` workgroups, n views of `tiles` tiles each among them, gives every XCD
+// neighbouring tiles: where most of the launch is on the device at once (f32 up to 8 workgroups a CU,
+// 16-bit types, whose rays wait less, 12) and the views are few, a tile's rays find little that an
+// earlier view fetched and more that the next tile does.  Measured dealt / in ranges (us): 100^3, 128^2
+// detector, 24 views f32 108 / 94, f16 107 / 82; 128^3, 200^2, 4 views f32 102 / 97, bf16 80 / 78, 16 views
+// bf16 157 / 142, f16 161 / 150; 256^3, 400^2, 2 views f32 257 / 245, bf16 208 / 199.  Beyond the lines: 192^3,
+// 300^2, 6 views f32 246 / 270, 256^3, 4 views 364 / 428; 64^3, 40 views bf16 60 / 63; more than 640 tiles
+// f16 384^3, 600^2, one view, 542 / 568.  Where the volume itself is sampled (DIRECT) the line is at 64
+// tiles: 100^3, 128^2, 24 views bf16 1392 / 1037; 128^3, 200^2, 8 views 1084 / 1321.
+template <typename TS, bool DIRECT = false> static bool fwd_neighbours(long long blocks, int n, long long tiles) {
+  return n <= 32 && tiles <= (DIRECT ? 64 : 640) && blocks <= (sizeof(TS) == 2 && !DIRECT ? 3072 : 2048);
+}
+
 // DIRECT: P.cells is the volume [D][H][W] itself, sampled with sample_direct.
 template <typename TS, bool HW, typename IT, bool DIRECT = false, typename TL = FwdTile16>
 __device__ __forceinline__ void fwd_block(const FwdProblem &P, long long q) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int xcd = (int)(q % kXcds);
   const long long qq = q / kXcds;  // view fastest, then the XCD's tiles
-  const long long k = qq / P.n;
-  const int view = (int)(qq - k * P.n);
-  const long long t = k * kXcds + xcd;
-  if (t >= (long long)P.tiles_x * P.tiles_y) return;
-  const int ty = (int)(t / P.tiles_x), tx = (int)(t - (long long)ty * P.tiles_x);
+  const int k = (int)(qq / P.n);
+  const int view = (int)(qq - (long long)k * P.n);
+  const int t = fwd_tile(k, xcd, view, P.n, P.tiles_x * P.tiles_y, P.neighbours);
+  if (t < 0) return;
+  const int ty = t / P.tiles_x, tx = t - ty * P.tiles_x;
   const int W = P.W, H = P.H, D = P.D, Hd = P.Hd, Wd = P.Wd;
   // Lanes past the detector's last column or row: in the 16-bit streamed march they march a
   // copy of the edge pixel's ray and store nothing, so that every lane of the wave takes
@@ -1244,10 +1276,11 @@ static void launch_fwd(bool hw, const void *cells, float *sino, const float *inv
   const long long cs = (long long)cell_elems<TS>(D, H, W);
   const bool small = fwd_small_index<TS>(D, H, W);
   const int per = fwd_views_per_launch(n, Hd, Wd);
+  const bool neighbours = fwd_neighbours<TS>(B * fwd_blocks(n, Hd, Wd), n, (long long)((Wd + 15) / 16) * ((Hd + 15) / 16));
   for (int v0 = 0; v0 < n; v0 += per) {
     const int k = n - v0 < per ? n - v0 : per;
     FwdProblem P{cells, sino + (size_t)v0 * Hd * Wd, inv_ar + (size_t)v0 * 9, src + (size_t)v0 * 3, step,
-                 spacing, W, H, D, k, Hd, Wd, (Wd + 15) / 16, (Hd + 15) / 16, 0};
+                 spacing, W, H, D, k, Hd, Wd, (Wd + 15) / 16, (Hd + 15) / 16, 0, neighbours};
     dim3 grid((unsigned)fwd_blocks(k, Hd, Wd), 1, B);
     if (fwd_byte_offsets<TS>(D, H, W))
       launch_fwd_it<TS, unsigned>(hw, P, grid, cs, n, stream);
@@ -1266,10 +1299,12 @@ static void launch_fwd_direct(bool hw, const void *vol, float *sino, const float
                               int H, int W, int n, int Hd, int Wd, hipStream_t stream) {
   const long long vs = (long long)D * H * W;
   const int per = fwd_views_per_launch(n, Hd, Wd);
+  const bool neighbours =
+      fwd_neighbours<TS, true>(B * fwd_blocks(n, Hd, Wd), n, (long long)((Wd + 15) / 16) * ((Hd + 15) / 16));
   for (int v0 = 0; v0 < n; v0 += per) {
     const int k = n - v0 < per ? n - v0 : per;
     FwdProblem P{vol, sino + (size_t)v0 * Hd * Wd, inv_ar + (size_t)v0 * 9, src + (size_t)v0 * 3, step,
-                 spacing, W, H, D, k, Hd, Wd, (Wd + 15) / 16, (Hd + 15) / 16, 0};
+                 spacing, W, H, D, k, Hd, Wd, (Wd + 15) / 16, (Hd + 15) / 16, 0, neighbours};
     dim3 grid((unsigned)fwd_blocks(k, Hd, Wd), 1, B);
     if (hw)
       cone_fwd_kernel<TS, true, long long, true><<<grid, dim3(256), 0, stream>>>(P, vs, n);
@@ -1777,11 +1812,13 @@ static int fwd_batched(const pyronn_cone_problem *pr, int count, bool hw, int bp
     bytes = bytes && fwd_byte_offsets<TS>(p.D, p.H, p.W);
     fb.p[k] = FwdProblem{cells, p.output, inv_ar, src, p.step_size, p.volume_spacing,
                          p.W, p.H, p.D, p.n_views, p.det_h, p.det_w,
-                         (p.det_w + tc - 1) / tc, (p.det_h + tr - 1) / tr, begin};
+                         (p.det_w + tc - 1) / tc, (p.det_h + tr - 1) / tr, begin, false};
     begin += fwd_blocks(p.n_views, p.det_h, p.det_w, tile);
   }
   fb.count = count;
   fb.total = begin;
+  for (int k = 0; k < count; ++k)
+    fb.p[k].neighbours = fwd_neighbours<TS>(begin, fb.p[k].n, (long long)fb.p[k].tiles_x * fb.p[k].tiles_y);
   // bpc <= 0: one workgroup per item (grid 0 below); else a persistent grid
   long long grid = 0;
   if (bpc > 0) {

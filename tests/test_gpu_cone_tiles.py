@@ -23,6 +23,35 @@ def test_forward_tiles_one_to_forty(det, storage):
     _check_views(vol, P, sp, og, det, 0.5, False, views=range(5))
 
 
+@pytest.mark.parametrize("det, n", [
+    ((16, 16), 1), ((20, 33), 8), ((33, 100), 32),     # ranges of neighbouring tiles: 1, 6, 21 of them
+    ((20, 33), 33), ((40, 16), 40), ((33, 100), 33),   # dealt, with a partial last turn
+    ((40, 120), 41), ((20, 250), 57), ((64, 60), 67),  # 8, 16 and 4 tile columns; partial groups of views
+    ((320, 512), 2), ((320, 513), 2),                  # 640 and 660 tiles
+])
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+def test_forward_tile_orders(det, n, storage):
+    shape = (20, 24, 18)
+    sp, og, P = _orbit(shape, n, 100.0, 160.0, det, (60.0 / det[0], 60.0 / det[1]))
+    vol = _rand_volume(shape, det[0], gh.DT[storage][1])
+    _check_views(vol, P, sp, og, det, 0.5, False, views=range(n))
+
+
+@pytest.mark.parametrize("blocks_per_cu", [0, 2])
+@pytest.mark.parametrize("views", [(4, 30), (40, 9), (33, 50)])   # all in ranges; too many views; too many blocks
+def test_batched_forward_tile_orders(views, blocks_per_cu):
+    det = [(40, 120), (100, 130)]
+    geoms = [geo.ConeGeometry((20, 24, 18), (1.0, 1.0, 1.0), d, (60.0 / d[0], 60.0 / d[1]), n, 100.0, 160.0, step_size=0.5)
+             for d, n in zip(det, views)]
+    vols = [_rand_volume((20, 24, 18), n) for n in views]
+    for tile in range(4):
+        got = batched.cone_projection3d_batched(vols, geoms, blocks_per_cu=blocks_per_cu, forward_tile=tile)
+        for x, v, g in zip(got, vols, geoms):
+            P = g.projection_matrices().astype(np.float32)
+            sp, og = np.asarray(g.volume_spacing, np.float32), np.asarray(g.volume_origin, np.float32)
+            assert np.array_equal(x.cpu().numpy(), gh.cone_forward(v.cpu().numpy(), P, sp, og, g.detector_shape, 0.5)[0])
+
+
 @pytest.mark.parametrize("det", [(512, 33), (497, 16), (528, 17), (496, 20), (640, 18)])
 @pytest.mark.parametrize("storage", ["bf16", "f16"])
 def test_forward_tile_rows_around_thirty_two(det, storage):
