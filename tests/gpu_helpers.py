@@ -107,6 +107,23 @@ def _geo2d(B, vo, do_, vs, ds, rays, n, sid=None, sdd=None):
     return g
 
 
+def _both2d(name, head, tail, shape, ws_bytes):
+    """The 2D entry that samples the data in place and, where there is one, the entry that samples a
+    copy in a workspace (what the operators call): both results must be the same."""
+    out = torch.full(shape, -7.25, device="cuda")
+    nat.call(name, *head, *tail, p(out), stream())
+    torch.cuda.synchronize()
+    res = out.cpu().numpy()
+    if ws_bytes:
+        work = torch.full((ws_bytes,), 0x7f, dtype=torch.uint8, device="cuda")
+        out = torch.full(shape, -7.25, device="cuda")
+        nat.call(name + "_ws", *head, *tail, p(out), p(work), ws_bytes, stream())
+        torch.cuda.synchronize()
+        copied = out.cpu().numpy()
+        assert np.array_equal(copied, res, equal_nan=True), f"{name}_ws: {int((copied != res).sum())} values differ"
+    return res
+
+
 def forward2d(fan, vol, rays, det, vo, vs, do_, ds, sid=None, sdd=None, step_factor=0.2, storage="f32"):
     vol = _batched(vol, 2)
     B, H, W = vol.shape
@@ -114,15 +131,11 @@ def forward2d(fan, vol, rays, det, vo, vs, do_, ds, sid=None, sdd=None, step_fac
     code, tdt = DT[storage]
     v = dev(vol, tdt)
     g = _geo2d(B, vo, do_, vs, ds, rays, n, sid, sdd)
-    out = torch.empty((B, n, det), device="cuda")
-    if fan:
-        nat.call("pyronn_fan_projection2d", p(v), code, B, H, W, p(g["vo"]), p(g["do"]), p(g["vs"]), p(g["ds"]),
-                 p(g["sid"]), p(g["sdd"]), p(g["rays"]), n, det, float(step_factor), p(out), stream())
-    else:
-        nat.call("pyronn_parallel_projection2d", p(v), code, B, H, W, p(g["vo"]), p(g["do"]), p(g["vs"]),
-                 p(g["ds"]), p(g["rays"]), n, det, float(step_factor), p(out), stream())
-    torch.cuda.synchronize()
-    return out.cpu().numpy()
+    head = [p(v), code, B, H, W, p(g["vo"]), p(g["do"]), p(g["vs"]), p(g["ds"])]
+    head += [p(g["sid"]), p(g["sdd"])] if fan else []
+    return _both2d("pyronn_fan_projection2d" if fan else "pyronn_parallel_projection2d", head,
+                   [p(g["rays"]), n, det, float(step_factor)], (B, n, det),
+                   nat.lib().pyronn_projection2d_workspace_size(B, H, W, code))
 
 
 def backward2d(fan, sino, rays, vol_shape, vo, vs, do_, ds, sid=None, sdd=None, storage="f32"):
@@ -132,15 +145,11 @@ def backward2d(fan, sino, rays, vol_shape, vo, vs, do_, ds, sid=None, sdd=None, 
     code, tdt = DT[storage]
     s_ = dev(sino, tdt)
     g = _geo2d(B, vo, do_, vs, ds, rays, n, sid, sdd)
-    out = torch.empty((B, H, W), device="cuda")
-    if fan:
-        nat.call("pyronn_fan_backprojection2d", p(s_), code, B, n, det, p(g["vo"]), p(g["do"]), p(g["vs"]),
-                 p(g["ds"]), p(g["sid"]), p(g["sdd"]), p(g["rays"]), H, W, p(out), stream())
-    else:
-        nat.call("pyronn_parallel_backprojection2d", p(s_), code, B, n, det, p(g["vo"]), p(g["do"]), p(g["vs"]),
-                 p(g["ds"]), p(g["rays"]), H, W, p(out), stream())
-    torch.cuda.synchronize()
-    return out.cpu().numpy()
+    head = [p(s_), code, B, n, det, p(g["vo"]), p(g["do"]), p(g["vs"]), p(g["ds"])]
+    head += [p(g["sid"]), p(g["sdd"])] if fan else []
+    return _both2d("pyronn_fan_backprojection2d" if fan else "pyronn_parallel_backprojection2d", head,
+                   [p(g["rays"]), H, W], (B, H, W),
+                   nat.lib().pyronn_backprojection2d_workspace_size(B, n, det, code))
 
 
 def parity(gpu, ref, rel_l2=1e-5, max_rel=1e-4):

@@ -234,3 +234,24 @@ def test_backprojection_detector_beyond_2_24_cells(storage, hw):
     ref, _ = orc.cone_backward(sq, P, shape, sp, og, hw=hw)
     assert np.abs(ref).max() > 0
     assert np.array_equal(rec, ref)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("det, floats", [((4094, 2044), True), ((4094, 2045), False), ((2046, 4094), False)])
+def test_backprojection_detector_around_2_23_cells(det, floats, storage):
+    """(H_d + 2)(W_d + 3) cells just below 2^23, where the offsets are formed in floats, at 2^23 and just
+    above, in integers.  The volume's shadow lies over the far corner of the detector."""
+    assert ((det[0] + 2) * (det[1] + 3) < 2 ** 23) == floats
+    shape = (16, 16, 16)
+    sp = np.ones(3, np.float32)
+    og = geo.centred_origin(shape, sp).astype(np.float32)
+    P = geo.circular_projection_matrices(2, 100.0, 200.0, det, (0.03, 0.03),
+                                         principal_point=(det[1] - 200.0, det[0] - 150.0)).astype(np.float32)
+    sino = np.random.default_rng(det[1]).uniform(0.0, 1.0, (2,) + det).astype(np.float32)
+    print(f"detector {det} {storage}", flush=True)
+    for tilt in (0.0, 1e-4):
+        P[:, 2, 2] += np.float32(tilt)
+        rec = gh.cone_backward(sino, P, sp, og, shape, storage=storage)[0]
+        ref, _ = orc.cone_backward(gh.quantise(sino, storage), P, shape, sp, og)
+        assert (ref != 0).any() and (ref == 0).any()     # partly off the detector
+        assert np.array_equal(rec, ref)

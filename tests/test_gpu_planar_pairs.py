@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+import gpu_helpers as gh
 import oracle as orc
 from pyronn_layers import geometry as geo
 from pyronn_layers import native as nat
@@ -156,3 +157,88 @@ def test_no_room_for_the_copy(back):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(got, want)
+
+
+def _mixed(B, H, W, n, det):
+    """Geometries of B items that differ in everything: spacings of every division, offsets, rays, radii."""
+    rng = np.random.default_rng(B * 1000 + H)
+    sp = np.array([(1.0, 1.0), (0.7, 1.3), (0.5, 0.25), (1e-19, 1e-19), (0.3, 0.3)], np.float32)
+    vs = sp[np.arange(B) % len(sp)]
+    ext = (np.array([H, W]) * vs).max(1)
+    vo = np.array([geo.centred_origin((H, W), v) for v in vs]) + rng.normal(size=(B, 2)) * ext[:, None] * 0.05
+    ds = np.where(np.arange(B) % 4 == 1, 2.0 ** np.round(np.log2(1.3 * ext / det)), 1.3 * ext / det)
+    do = -(det - 1) / 2 * ds + rng.normal(size=B) * ds
+    rays = np.stack([geo.parallel_ray_vectors(n, 1.0 + b) for b in range(B)])
+    f = lambda a: np.asarray(a, np.float32)
+    return f(vo), f(do), f(vs), f(ds), f(rays), f(1.6 * ext), f(2.1 * ext)
+
+
+@pytest.mark.parametrize("fan", [False, True])
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+@pytest.mark.parametrize("B, H, W, n, det", [
+    (5, 19, 23, 7, 31),        # 16 lanes per ray
+    (6, 33, 31, 50, 90),       # 8
+    (6, 17, 12, 110, 101),     # 4
+    (41, 5, 6, 3, 9),          # several rows and items per layout block
+])
+def test_batches_of_different_items(fan, storage, B, H, W, n, det):
+    vo, do, vs, ds, rays, sid, sdd = _mixed(B, H, W, n, det)
+    rng = np.random.default_rng(B)
+    img = gh.quantise(rng.normal(size=(B, H, W)), storage)
+    sino = gh.quantise(rng.normal(size=(B, n, det)), storage)
+    # one step for the launch: a step of half a spacing
+    fwd = gh.forward2d(fan, img, rays, det, vo, vs, do, ds, sid, sdd, 0.5, storage)
+    back = gh.backward2d(fan, sino, rays, (H, W), vo, vs, do, ds, sid, sdd, storage)
+    for b in range(B):
+        if fan:
+            ref = orc.fan_forward(img[b], rays[b], det, vo[b], vs[b], do[b], ds[b], sid=sid[b], sdd=sdd[b], step_factor=0.5)[0]
+            rb = orc.fan_backward(sino[b], rays[b], (H, W), vo[b], vs[b], do[b], ds[b], sid=sid[b], sdd=sdd[b])
+        else:
+            ref = orc.parallel_forward(img[b], rays[b], det, vo[b], vs[b], do[b], ds[b], step_factor=0.5)[0]
+            rb = orc.parallel_backward(sino[b], rays[b], (H, W), vo[b], vs[b], do[b], ds[b])
+        rb = rb[0] if isinstance(rb, tuple) else rb
+        assert np.array_equal(fwd[b], ref, equal_nan=True), f"forward, item {b}"
+        assert np.array_equal(back[b], rb, equal_nan=True), f"backward, item {b}"
+
+
+def test_more_pixels_than_a_round_of_blocks_in_a_batch():
+    B, H, W, n, det = 40, 112, 117, 6, 160      # 2240 blocks
+    vo, do, vs, ds, rays, sid, sdd = _mixed(B, H, W, n, det)
+    sino = np.random.default_rng(2).normal(size=(B, n, det)).astype(np.float32)
+    back = gh.backward2d(True, sino, rays, (H, W), vo, vs, do, ds, sid, sdd)
+    for b in (0, 1, 2, 3, 17, 39):
+        rb = orc.fan_backward(sino[b], rays[b], (H, W), vo[b], vs[b], do[b], ds[b], sid=sid[b], sdd=sdd[b])
+        assert np.array_equal(back[b], rb[0] if isinstance(rb, tuple) else rb, equal_nan=True), f"item {b}"
+
+
+@pytest.mark.parametrize("fan", [False, True])
+@pytest.mark.parametrize("name", ["vo", "do", "ds", "rays"])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_geometry_that_is_not_finite(fan, name, value):
+    # one item of a batch of two: same values from the copy and in place, the other item untouched by it
+    H, W, n, det = 12, 14, 6, 20
+    vo, do, vs, ds, rays, sid, sdd = _mixed(2, H, W, n, det)
+    bad = {"vo": vo, "do": do, "ds": ds, "rays": rays}[name]
+    bad.reshape(2, -1)[1, 0] = value
+    rng = np.random.default_rng(1)
+    img, sino = rng.normal(size=(2, H, W)).astype(np.float32), rng.normal(size=(2, n, det)).astype(np.float32)
+    fwd = gh.forward2d(fan, img, rays, det, vo, vs, do, ds, sid, sdd, 0.5)
+    back = gh.backward2d(fan, sino, rays, (H, W), vo, vs, do, ds, sid, sdd)
+    assert np.isfinite(fwd[0]).all() and np.isfinite(back[0]).all()
+
+
+@pytest.mark.parametrize("det, copied", [(2 ** 22 - 1, True), (2 ** 22, False)])
+@pytest.mark.parametrize("fan", [False, True])
+def test_rows_longest_detector_and_the_first_past_it(fan, det, copied):
+    assert (nat.lib().pyronn_backprojection2d_workspace_size(1, 3, det, nat.F32) > 0) == copied
+    rng = np.random.default_rng(det)
+    sino = rng.normal(size=(3, det)).astype(np.float32)
+    H, W = 9, 2100
+    vs, vo = np.ones(2, np.float32), geo.centred_origin((H, W), (1.0, 1.0)).astype(np.float32)
+    ds = np.float32(2.0 ** -11)                     # the pixels reach both ends of the detector
+    do = np.float32(-(det - 1) / 2 * float(ds))
+    rays = geo.parallel_ray_vectors(3, math.pi).astype(np.float32)
+    kw = dict(sid=np.float32(9000.0), sdd=np.float32(9500.0)) if fan else {}
+    back = gh.backward2d(fan, sino, rays, (H, W), vo, vs, do, ds, **kw)
+    ref = (orc.fan_backward if fan else orc.parallel_backward)(sino, rays, (H, W), vo, vs, do, ds, **kw)
+    assert np.array_equal(back[0], ref[0] if isinstance(ref, tuple) else ref)
