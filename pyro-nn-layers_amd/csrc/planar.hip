@@ -286,13 +286,24 @@ template <> struct PairLoad<float> {
 __host__ __device__ inline int pair_cols(int W) { return W + 4; }
 __host__ __device__ inline int pair_rows(int H) { return H + 3; }
 
-// One lane per element.
+// Lanes of a 256-lane layout block that share a row of `cols` elements, log2: a block takes several short
+// rows, as one each would leave most of its lanes idle and the launch bound by its blocks (a parallel
+// projection of a 65000 x 4 image 34 -> 8 us; a backprojection of 8 views to 4096 images of 8 x 8, with one
+// pixel per lane, 30 -> 12).
+static int layout_lanes(int cols) {
+  int s = 3;
+  while (s < 8 && (1 << s) < cols) ++s;
+  return s;
+}
+
+// One lane per element, 1 << lanes columns of 256 >> lanes rows per block.
 template <typename TS>
 __global__ void __launch_bounds__(256)
-build_pairs_kernel(const TS *__restrict__ img, TS *__restrict__ pairs, int H, int W) {
-  const int cx = blockIdx.x * 256 + threadIdx.x, cy = blockIdx.y;
+build_pairs_kernel(const TS *__restrict__ img, TS *__restrict__ pairs, int H, int W, int lanes) {
+  const int cx = (blockIdx.x << lanes) + (threadIdx.x & ((1 << lanes) - 1));
+  const int cy = blockIdx.y * (256 >> lanes) + (threadIdx.x >> lanes);
   const int Wp = pair_cols(W);
-  if (cx >= Wp) return;
+  if (cx >= Wp || cy >= pair_rows(H)) return;
   const TS *im = img + (size_t)blockIdx.z * H * W;
   const int x = cx - 2, y = cy - 2;
   const bool vx = x >= 0 && x < W;
@@ -696,22 +707,28 @@ back2d_kernel(const TS *__restrict__ sino, float *__restrict__ vol, const float 
 // forms the per-view terms once, in LDS (kBackViews views at a time; every lane reads them
 // back with two broadcast reads), both quotients share one correctly rounded reciprocal
 // (div_spacing's two corrections), and rcp_sqrt_fast serves the weight: about 68 per update.
-// The parallel kernel's 15 leave it to the address path, one pair load per update.  512^2 fan,
-// 360 views x 725: 221 -> 126 us (8 images 1233 -> 829); 256^2 parallel, 180 views x 363: 45 ->
-// 23.5 us (32 images 309 -> 181).  A test per view for the rare distances that rcp_sqrt_fast does
-// not serve kept the views' chains from overlapping: 52 x 48 fan, 44 views, 25.5 us with it (24.9
-// for back2d_kernel), 14 without.
+// The parallel kernel's 15 leave it to the address path, one pair load per update.  With the
+// layout pass, 512^2 fan, 360 views x 725: 239 -> 135 us (8 images 1431 -> 872); 256^2 parallel, 180
+// views x 363: 49.5 -> 26 us (32 images 327 -> 178).  A test per view for the rare distances that
+// rcp_sqrt_fast does not serve kept the views' chains from overlapping: 52 x 48 fan, 44 views, 25.5 us
+// with it (24.9 for back2d_kernel), 14 without.
 // =====================================================================================
 __host__ __device__ inline int row_len(int det) { return det + 4; }
 
+// 1 << lanes columns of 256 >> lanes rows per block and step (layout_lanes), four steps' loads in flight and
+// kRowsBlocks blocks at most, a device's worth: a copy of 189 MB (32 x 720 x 2048 f32) with one row per
+// block took about 150 us, now about 100.
+constexpr long long kRowsBlocks = 8192;
 template <typename TS>
 __global__ void __launch_bounds__(256)
-build_rows_kernel(const TS *__restrict__ sino, TS *__restrict__ rows, int det, long long nrows) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
+build_rows_kernel(const TS *__restrict__ sino, TS *__restrict__ rows, int det, long long nrows, int lanes) {
+  const int c = (blockIdx.x << lanes) + (threadIdx.x & ((1 << lanes) - 1));
   if (c >= row_len(det)) return;
   const int u = c - 2;
   const bool in = u >= 0 && u < det;
-  for (long long r = blockIdx.y; r < nrows; r += gridDim.y)
+  const int per = 256 >> lanes;
+#pragma unroll 4
+  for (long long r = (long long)blockIdx.y * per + (threadIdx.x >> lanes); r < nrows; r += (long long)gridDim.y * per)
     rows[(size_t)r * row_len(det) + c] = in ? sino[(size_t)r * det + u] : zero_of<TS>();
 }
 
@@ -774,10 +791,10 @@ __device__ __forceinline__ void fan_pixel(const ViewTerms &v, float pcx, float p
   dw = SQRT ? rcp_sqrt_fast(t) : rcp_rn(sqrtf(t));
 }
 
-template <typename TS, bool FAN, bool FAST, int DIV, int P>
+template <typename TS, bool FAN, bool FAST, int DIV>
 __device__ __forceinline__ void back2d_rows(const TS *__restrict__ rows, const float *__restrict__ rb, int n, int det,
-                                            float pcx, const float *pcy, float do_, float ds, float ids, float sid,
-                                            float sdd, ViewTerms *terms, float *val) {
+                                            float pcx, float pcy, float do_, float ds, float ids, float sid, float sdd,
+                                            ViewTerms *terms, float &val) {
   const float fdet = (float)det;
   constexpr uint32_t bias = 0x4B000000u << (sizeof(TS) == 4 ? 2 : 1);
   const char *base = reinterpret_cast<const char *>(rows) - (size_t)bias;
@@ -811,55 +828,46 @@ __device__ __forceinline__ void back2d_rows(const TS *__restrict__ rows, const f
       // U views at a time without a branch between them, so that their chains and loads overlap:
       // one test for all of them that rcp_sqrt_fast serves every distance (a NaN passes and
       // stays one)
-      constexpr int U = 4 / P;
+      constexpr int U = 4;
       int k = 0;
       for (; FAST && near && k + U <= nv; k += U, base += U * row_bytes) {
         float closest = 1.0f;
 #pragma unroll
-        for (int j = 0; j < U; ++j)
-#pragma unroll
-          for (int p = 0; p < P; ++p) closest = fminf(closest, fan_distance2(terms[k + j], pcx, pcy[p]));
+        for (int j = 0; j < U; ++j) closest = fminf(closest, fan_distance2(terms[k + j], pcx, pcy));
         if (!__all(closest >= 0x1p-100f)) break;
 #pragma unroll
         for (int j = 0; j < U; ++j) {
-          const ViewTerms t = terms[k + j];
-#pragma unroll
-          for (int p = 0; p < P; ++p) {
-            float s, dw;
-            fan_pixel<true, true>(t, pcx, pcy[p], s, dw);
-            const float f = sample_row<TS>(base + j * row_bytes, fdet, div_spacing<DIV>(s - do_, ds, ids));
-            val[p] = fmaf(f * dw, dw, val[p]);
-          }
+          const ViewTerms t = terms[k + j];  // in registers: 136 us for one 512^2 image, 145 read where used
+          float s, dw;
+          fan_pixel<true, true>(t, pcx, pcy, s, dw);
+          const float f = sample_row<TS>(base + j * row_bytes, fdet, div_spacing<DIV>(s - do_, ds, ids));
+          val = fmaf(f * dw, dw, val);
         }
       }
       for (; k < nv; ++k, base += row_bytes) {
         const ViewTerms t = terms[k];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-          float s, dw;
-          fan_pixel<FAST, false>(t, pcx, pcy[p], s, dw);
-          const float f = sample_row<TS>(base, fdet, div_spacing<DIV>(s - do_, ds, ids));
-          val[p] = fmaf(f * dw, dw, val[p]);
-        }
+        float s, dw;
+        fan_pixel<FAST, false>(t, pcx, pcy, s, dw);
+        const float f = sample_row<TS>(base, fdet, div_spacing<DIV>(s - do_, ds, ids));
+        val = fmaf(f * dw, dw, val);
       }
     } else {
 #pragma unroll 4  // four views in flight: each load would be waited for alone
       for (int k = 0; k < nv; ++k, base += row_bytes) {
         const float c0 = terms[k].srx, m1 = pcx * terms[k].sry;
-#pragma unroll
-        for (int p = 0; p < P; ++p)
-          val[p] += sample_row<TS>(base, fdet, div_spacing<DIV>(fmaf(pcy[p], c0, m1) - do_, ds, ids));
+        val += sample_row<TS>(base, fdet, div_spacing<DIV>(fmaf(pcy, c0, m1) - do_, ds, ids));
       }
     }
   }
 }
 
-// P pixels per lane, 16 rows apart; a block covers 16 x 16 P pixels.  FAST holds when the
+// One pixel per lane, 16 x 16 pixels per block (two pixels 16 rows apart took 10 to 47% longer: 6 fan images
+// of 301 x 277, 185 against 161 us; 400 of 40 x 40 301 against 226).  FAST holds when the
 // detector spacing lies in [2^-30, 2^30] and every length of the geometry below 2^20 mm: the
 // denominator (at least 1e-6 where it is used) and the quotients then stay far inside the
 // range of the refined division, and a quotient so small that its residual is inexact
 // vanishes in the sampler's + 0.5.  The choices are uniform over the block and change no bit.
-template <typename TS, bool FAN, int P>
+template <typename TS, bool FAN>
 __global__ void __launch_bounds__(256)
 back2d_rows_kernel(const TS *__restrict__ rows, float *__restrict__ vol, const float *__restrict__ rays,
                    const float *__restrict__ vorigin, const float *__restrict__ dorigin,
@@ -867,18 +875,12 @@ back2d_rows_kernel(const TS *__restrict__ rows, float *__restrict__ vol, const f
                    const float *__restrict__ sid_p, const float *__restrict__ sdd_p, int H, int W, int n, int det) {
   __shared__ ViewTerms terms[kBackViews];
   const int x = blockIdx.x * 16 + (threadIdx.x & 15);
-  const int y = blockIdx.y * 16 * P + (threadIdx.x >> 4);
+  const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
   const int b = blockIdx.z;
   const float sx = vspacing[b * 2 + 1], sy = vspacing[b * 2 + 0];
   const float ox = vorigin[b * 2 + 1], oy = vorigin[b * 2 + 0];
   const float do_ = dorigin[b], ds = dspacing[b];
-  const float pcx = i2p((float)x, ox, sx);
-  float pcy[P], val[P];
-#pragma unroll
-  for (int p = 0; p < P; ++p) {
-    pcy[p] = i2p((float)(y + 16 * p), oy, sy);
-    val[p] = 0.0f;
-  }
+  const float pcx = i2p((float)x, ox, sx), pcy = i2p((float)y, oy, sy);
   const float *rb = rays + (size_t)b * n * 2;
   rows += (size_t)b * n * row_len(det);
   float sid = 0.0f, sdd = 0.0f;
@@ -889,21 +891,17 @@ back2d_rows_kernel(const TS *__restrict__ rows, float *__restrict__ vol, const f
   const float pow2 = pow2_reciprocal(ds);
   const float far = fmaxf(fmaxf(fabsf(sid), fabsf(sdd)),
                           fmaxf(fmaxf(fabsf(ox), fabsf(i2p((float)(W + 16), ox, sx))),
-                                fmaxf(fabsf(oy), fabsf(i2p((float)(H + 16 * P), oy, sy)))));
+                                fmaxf(fabsf(oy), fabsf(i2p((float)(H + 16), oy, sy)))));
   const bool fast = ds >= 0x1p-30f && ds <= 0x1p30f && far < 0x1p20f;
+  float val = 0.0f;
   if (!fast)
-    back2d_rows<TS, FAN, false, kDivIeee, P>(rows, rb, n, det, pcx, pcy, do_, ds, 0.0f, sid, sdd, terms, val);
+    back2d_rows<TS, FAN, false, kDivIeee>(rows, rb, n, det, pcx, pcy, do_, ds, 0.0f, sid, sdd, terms, val);
   else if (pow2 != 0.0f)
-    back2d_rows<TS, FAN, true, kDivPow2, P>(rows, rb, n, det, pcx, pcy, do_, ds, pow2, sid, sdd, terms, val);
+    back2d_rows<TS, FAN, true, kDivPow2>(rows, rb, n, det, pcx, pcy, do_, ds, pow2, sid, sdd, terms, val);
   else
-    back2d_rows<TS, FAN, true, kDivRefine, P>(rows, rb, n, det, pcx, pcy, do_, ds, 1.0f / ds, sid, sdd, terms, val);
-#pragma unroll
-  for (int p = 0; p < P; ++p) {
-    if (x < W && y + 16 * p < H) {
-      float *o = vol + ((size_t)b * H + (y + 16 * p)) * W + x;
-      *o = FAN ? (((sid * sdd) * kPi) * val[p]) / (float)n : (kPi * val[p]) / (float)n;
-    }
-  }
+    back2d_rows<TS, FAN, true, kDivRefine>(rows, rb, n, det, pcx, pcy, do_, ds, 1.0f / ds, sid, sdd, terms, val);
+  if (x < W && y < H)
+    vol[((size_t)b * H + y) * W + x] = FAN ? (((sid * sdd) * kPi) * val) / (float)n : (kPi * val) / (float)n;
 }
 
 // rays per launch below which a ray gets four lanes
@@ -938,8 +936,10 @@ static void launch_pairs(const void *volume, int batch, int H, int W, const floa
                          const float *vs, const float *ds, const float *sid, const float *sdd, const float *rays, int n,
                          int det, float step_factor, float *sino, void *ws, hipStream_t s) {
   TS *pairs = (TS *)ws;
-  build_pairs_kernel<TS><<<dim3((unsigned)((pair_cols(W) + 255) / 256), (unsigned)pair_rows(H), (unsigned)batch),
-                           dim3(256), 0, s>>>((const TS *)volume, pairs, H, W);
+  const int lanes = layout_lanes(pair_cols(W)), per = 256 >> lanes;
+  build_pairs_kernel<TS><<<dim3((unsigned)((pair_cols(W) + (1 << lanes) - 1) >> lanes),
+                                (unsigned)((pair_rows(H) + per - 1) / per), (unsigned)batch),
+                           dim3(256), 0, s>>>((const TS *)volume, pairs, H, W, lanes);
   const long long nrays = (long long)det * n * batch;
   const int G = nrays < kRowRays ? 16 : nrays < kHalfRowRays ? 8 : 4;
   // one wave per block: the rays of a view differ in length, and the dispatch evens out
@@ -1006,20 +1006,13 @@ static void launch_rows(const void *sino, int batch, int n, int det, const float
                         int W, float *vol, void *ws, hipStream_t s) {
   TS *rows = (TS *)ws;
   const long long nrows = (long long)batch * n;
-  build_rows_kernel<TS><<<dim3((unsigned)((row_len(det) + 255) / 256), (unsigned)(nrows < 32768 ? nrows : 32768)),
-                          dim3(256), 0, s>>>((const TS *)sino, rows, det, nrows);
-  // One pixel per lane while the blocks fit the device at once (8 of 256 lanes per CU), two
-  // beyond: a few blocks past a full round run alone for as long as the round did (6 fan images
-  // of 301 x 277, 2052 blocks: 264 against 184 us), below it the second pixel only lengthens a
-  // block (512^2, 1024 blocks: 133 against 148).
-  const long long blocks = (long long)((W + 15) / 16) * ((H + 15) / 16) * batch;
-  if (blocks <= 2048) {
-    const dim3 grid((W + 15) / 16, (H + 15) / 16, batch);
-    back2d_rows_kernel<TS, FAN, 1><<<grid, dim3(256), 0, s>>>(rows, vol, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det);
-  } else {
-    const dim3 grid((W + 15) / 16, (H + 31) / 32, batch);
-    back2d_rows_kernel<TS, FAN, 2><<<grid, dim3(256), 0, s>>>(rows, vol, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det);
-  }
+  const int lanes = layout_lanes(row_len(det)), per = 256 >> lanes;
+  const long long gx = (row_len(det) + (1 << lanes) - 1) >> lanes, need = (nrows + per - 1) / per;
+  const long long most = gx < kRowsBlocks ? kRowsBlocks / gx : 1;
+  build_rows_kernel<TS><<<dim3((unsigned)gx, (unsigned)(need < most ? need : most)), dim3(256), 0, s>>>(
+      (const TS *)sino, rows, det, nrows, lanes);
+  const dim3 grid((W + 15) / 16, (H + 15) / 16, batch);
+  back2d_rows_kernel<TS, FAN><<<grid, dim3(256), 0, s>>>(rows, vol, rays, vo, dor, vs, ds, sid, sdd, H, W, n, det);
 }
 
 template <bool FAN>

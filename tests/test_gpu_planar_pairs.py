@@ -1,6 +1,6 @@
 """The 2D projections through the pair copy of the images and the 2D backprojections through the
 bordered copy of the projections: the dispatch's edges (lanes per ray, remainders of the ray
-groups, pixels per lane, spacings of each division, the largest copy) against the oracle."""
+groups, rows of the copies, spacings of each division, the largest copy) against the oracle."""
 import math
 
 import numpy as np
@@ -109,7 +109,7 @@ def _back(fan, sino, shape, sp, ds, sid, storage=torch.float32, off=(0.0, 0.0)):
     ((17, 15), (0.7, 1.3), 7, 2, 9.0),        # a detector of one cell; refined division
     ((33, 47), (1.0, 1.0), 129, 65, 0.5),     # one view past a block's table of 128
     ((30, 31), (0.3, 0.3), 256, 40, 0.25),    # a detector smaller than the shadow
-    ((728, 730), (1.0, 1.0), 6, 911, 1.7),    # 2116 blocks: two pixels per lane, ragged rows
+    ((728, 730), (1.0, 1.0), 6, 911, 1.7),    # 2116 blocks, ragged rows
     ((20, 20), (1.0, 1.0), 5, 30, 1e-12),     # a spacing outside the refined division's range
 ])
 def test_rows_match_the_oracle(fan, storage, shape, sp, n, det, ds):
@@ -199,6 +199,34 @@ def test_batches_of_different_items(fan, storage, B, H, W, n, det):
         rb = rb[0] if isinstance(rb, tuple) else rb
         assert np.array_equal(fwd[b], ref, equal_nan=True), f"forward, item {b}"
         assert np.array_equal(back[b], rb, equal_nan=True), f"backward, item {b}"
+
+
+@pytest.mark.parametrize("n, det", [
+    (1, 1), (70, 4),               # 8 lanes a row of the copy: one row and blocks partly filled
+    (33, 12), (17, 13),            # 16, all of them used, and 32
+    (9, 124), (9, 125),            # 128 and 256
+    (5, 252), (5, 253),            # one and two blocks a row
+    (9000, 2), (700, 600),         # more row blocks than are launched at once: several steps each
+])
+def test_rows_of_every_length(n, det):
+    H, W = 5, 7
+    vo, do, vs, ds, rays, sid, sdd = _mixed(2, H, W, n, det)
+    sino = gh.quantise(np.random.default_rng(det).normal(size=(2, n, det)), "bf16")
+    back = gh.backward2d(False, sino, rays, (H, W), vo, vs, do, ds, storage="bf16")
+    for b in range(2):
+        ref = orc.parallel_backward(sino[b], rays[b], (H, W), vo[b], vs[b], do[b], ds[b])
+        assert np.array_equal(back[b], ref[0] if isinstance(ref, tuple) else ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("H, W", [(1, 4), (30, 4), (61, 12), (29, 28), (13, 252), (14, 253), (65532, 1)])
+def test_pairs_of_every_width(H, W):
+    vo, do, vs, ds, rays, sid, sdd = _mixed(2, H, W, 3, 40)
+    img = gh.quantise(np.random.default_rng(W).normal(size=(2, H, W)), "f16")
+    vs[:], ds[:] = 1.0, 1.3 * max(H, W) / 40
+    fwd = gh.forward2d(False, img, rays, 40, vo, vs, do, ds, step_factor=0.5, storage="f16")
+    for b in range(2):
+        ref = orc.parallel_forward(img[b], rays[b], 40, vo[b], vs[b], do[b], ds[b], step_factor=0.5)[0]
+        assert np.array_equal(fwd[b], ref)
 
 
 def test_more_pixels_than_a_round_of_blocks_in_a_batch():
