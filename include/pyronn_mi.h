@@ -212,9 +212,12 @@ int pyronn_fan_projection2d(const void *volume, int volume_dtype, int batch, int
  * The two 2D projections through a copy of the images in the workspace, laid out so that a
  * sample is one load: the same results as the calls above bit for bit, in a fraction of
  * their time.  pyronn_projection2d_workspace_size gives 0 where there is no such copy
- * ((W + 4)(H + 3) of 2^23 or more, H above 65532); use the calls above there.
+ * ((W + 4)(H + 3) of 2^23 or more, H above 65532); use the calls above there.  They are the faster
+ * ones where pyronn_projection2d_copy_pays gives 0: short rays, few rays over many pixels.
  */
 size_t pyronn_projection2d_workspace_size(int batch, int H, int W, int volume_dtype);
+int pyronn_projection2d_copy_pays(int batch, int H, int W, int volume_dtype, int n_views, int det,
+                                  float step_factor);
 int pyronn_parallel_projection2d_ws(const void *volume, int volume_dtype, int batch, int H, int W,
                                     const float *volume_origin, const float *detector_origin,
                                     const float *volume_spacing, const float *detector_spacing,
@@ -248,9 +251,12 @@ int pyronn_fan_backprojection2d(const void *sinogram, int sinogram_dtype, int ba
  * The two 2D backprojections through a copy of the projections with a zero border in the
  * workspace: the same results as the calls above bit for bit, faster.
  * pyronn_backprojection2d_workspace_size gives 0 for 2^22 detector pixels or more; use the
- * calls above there.
+ * calls above there.  They are the faster ones where pyronn_backprojection2d_copy_pays gives 0:
+ * few views, long projections to few pixels.
  */
 size_t pyronn_backprojection2d_workspace_size(int batch, int n_views, int det, int sinogram_dtype);
+int pyronn_backprojection2d_copy_pays(int fan, int batch, int n_views, int det, int sinogram_dtype,
+                                      int H, int W);
 int pyronn_parallel_backprojection2d_ws(const void *sinogram, int sinogram_dtype, int batch,
                                         int n_views, int det, const float *volume_origin,
                                         const float *detector_origin, const float *volume_spacing,

@@ -161,7 +161,7 @@ Geo2D geo2d(int64_t B, int64_t n, const at::Tensor &vo, const at::Tensor &dor, c
   return g;
 }
 
-// Workspace of the 2D operators' copies.  Undefined where there is no copy (0 bytes) and where the
+// Workspace of the 2D operators' copies.  Undefined where no copy is made (0 bytes) and where the
 // device has no room for it: the operators then sample the data as it lies, same bits, slower.
 at::Tensor copy_workspace(size_t bytes, const at::Tensor &data) {
   if (!bytes) return at::Tensor();
@@ -187,8 +187,10 @@ at::Tensor proj2d(bool fan, const at::Tensor &volume, at::IntArrayRef projection
   const int dt = dtype_code(vol, op);
   at::Tensor out = at::empty({B, n, det}, vol.options().dtype(at::kFloat));
   if (empty_output(out)) return out;
-  // the pair copy of the images that the projection samples; none for images too large for it
-  const size_t ws = pyronn_projection2d_workspace_size((int)B, (int)H, (int)W, dt);
+  // the pair copy of the images that the projection samples; none for images too large for it and where
+  // sampling the images as they lie is faster
+  const bool copy = pyronn_projection2d_copy_pays((int)B, (int)H, (int)W, dt, (int)n, (int)det, (float)step_size) != 0;
+  const size_t ws = copy ? pyronn_projection2d_workspace_size((int)B, (int)H, (int)W, dt) : 0;
   const at::Tensor work = copy_workspace(ws, vol);
   const float *vop = g.vo.data_ptr<float>(), *dop = g.dor.data_ptr<float>(), *vsp = g.vs.data_ptr<float>(),
               *dsp = g.ds.data_ptr<float>(), *rp = g.rays.data_ptr<float>();
@@ -227,8 +229,9 @@ at::Tensor back2d(bool fan, const at::Tensor &sinogram, at::IntArrayRef volume_s
   const int dt = dtype_code(sino, op);
   at::Tensor out = at::empty({B, H, W}, sino.options().dtype(at::kFloat));
   if (empty_output(out)) return out;
-  // the bordered copy of the projections that the backprojection samples
-  const size_t ws = pyronn_backprojection2d_workspace_size((int)B, (int)n, (int)det, dt);
+  // the bordered copy of the projections that the backprojection samples, on the same terms
+  const bool copy = pyronn_backprojection2d_copy_pays(fan, (int)B, (int)n, (int)det, dt, (int)H, (int)W) != 0;
+  const size_t ws = copy ? pyronn_backprojection2d_workspace_size((int)B, (int)n, (int)det, dt) : 0;
   const at::Tensor work = copy_workspace(ws, sino);
   const float *vop = g.vo.data_ptr<float>(), *dop = g.dor.data_ptr<float>(), *vsp = g.vs.data_ptr<float>(),
               *dsp = g.ds.data_ptr<float>(), *rp = g.rays.data_ptr<float>();

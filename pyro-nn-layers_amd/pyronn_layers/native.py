@@ -54,6 +54,7 @@ _SIGS = {
     "pyronn_fan_projection2d": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f,
                                      _vp, _vp]),
     "pyronn_projection2d_workspace_size": (_sz, [_i, _i, _i, _i]),
+    "pyronn_projection2d_copy_pays": (_i, [_i, _i, _i, _i, _i, _i, _f]),
     "pyronn_parallel_projection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp,
                                              _vp, _sz, _vp]),
     "pyronn_fan_projection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f,
@@ -61,6 +62,7 @@ _SIGS = {
     "pyronn_fan_backprojection2d": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,
                                          _vp, _vp]),
     "pyronn_backprojection2d_workspace_size": (_sz, [_i, _i, _i, _i]),
+    "pyronn_backprojection2d_copy_pays": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "pyronn_parallel_backprojection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp,
                                                  _vp, _sz, _vp]),
     "pyronn_fan_backprojection2d_ws": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,

@@ -247,3 +247,25 @@ def test_noalloc_forward_checks_arguments_before_any_device_call():
     rc = L.pyronn_cone_projection3d_noalloc(_fake(), 5, 1, 4, 4, 4, _fake(), _fake(), _fake(), _fake(), _fake(), 2,
                                             4, 4, 0, _fake(), None)
     assert rc == 1 and "dtype" in nat.last_error()
+
+
+def test_copies_of_the_2d_calls_are_made_where_they_pay():
+    f, b = nat.lib().pyronn_projection2d_copy_pays, nat.lib().pyronn_backprojection2d_copy_pays
+    F32, F16 = nat.F32, nat.F16
+    # forward: batch, H, W, dtype, views, det, step
+    assert f(1, 256, 256, F32, 180, 363, 0.2) and f(2, 64, 64, F32, 60, 95, 0.2) and f(1, 40, 40, F16, 40, 60, 0.5)
+    assert not f(1, 30, 30, F32, 8, 40, 1.0) and f(1, 31, 31, F32, 8, 40, 1.0)      # 30 samples of 0.11 us are 3.3 us
+    assert not f(256, 128, 128, F32, 1, 8, 1.0) and f(256, 128, 128, F16, 1, 8, 1.0)  # few rays, many pixels
+    assert f(4096, 8, 8, F32, 4, 11, 1.0) and not f(256, 8, 8, F32, 4, 11, 1.0)     # many short rays
+    assert not f(1, 4096, 4096, F32, 100, 100, 0.5)                                  # no copy to make
+    assert not f(1, 64, 64, F32, 0, 95, 0.2) and not f(1, 64, 64, F32, 60, 95, float("nan"))
+    # backward: fan, batch, views, det, dtype, H, W
+    for fan in (0, 1):
+        assert b(fan, 1, 360, 725, F32, 512, 512) and b(fan, 2, 60, 95, F32, 64, 64) and b(fan, 1, 40, 60, F16, 40, 40)
+        assert not b(fan, 1, 1, 725, F32, 512, 512) and not b(fan, 1, 4, 95, F16, 64, 64)
+        assert not b(fan, 1, 0, 95, F32, 64, 64) and not b(fan, 1, 60, 1 << 22, F32, 64, 64)
+    assert not b(0, 1, 27, 95, F32, 64, 64) and b(0, 1, 28, 95, F32, 64, 64)         # 28 (118 + 0.7 - 0.2) ns
+    assert not b(1, 1, 16, 95, F32, 64, 64) and b(1, 1, 17, 95, F32, 64, 64)
+    assert not b(0, 32, 720, 2048, F32, 16, 16) and b(0, 32, 720, 2048, F16, 16, 16)  # long rows, few pixels
+    # sizes that overflow 32 bits
+    assert b(1, 65535, 65535, 4000000, F16, 65535, 65535) in (0, 1) and f(65535, 1000, 8000, F32, 65535, 1 << 28, 1e-30)

@@ -33,6 +33,10 @@ def _run(fan, img, sp, n, det, ds, step, sid, storage=torch.float32, arc=2 * mat
         out = pl.parallel_projection2d(x, [n, det], *geom, dev(rays)[None], step)
         ref = orc.parallel_forward(x[0].float().cpu().numpy(), rays, det, org, sp, do, np.float32(ds),
                                    step_factor=step)[0]
+    # both entries, whichever of them the operator took
+    both = gh.forward2d(fan, x.float().cpu().numpy(), rays, det, org, sp, do, np.float32(ds), sid, 1.4 * sid, step,
+                        {torch.float32: "f32", torch.bfloat16: "bf16", torch.float16: "f16"}[storage])
+    assert np.array_equal(both[0], out[0].cpu().numpy(), equal_nan=True)
     return out[0].cpu().numpy(), ref
 
 
@@ -99,6 +103,9 @@ def _back(fan, sino, shape, sp, ds, sid, storage=torch.float32, off=(0.0, 0.0)):
     else:
         out = pl.parallel_backprojection2d(x, list(shape), *geom, dev(rays)[None])
         ref = orc.parallel_backward(s, rays, shape, org, sp, do, np.float32(ds))
+    both = gh.backward2d(fan, s[None], rays, shape, org, sp, do, np.float32(ds), sid, 1.4 * sid,
+                         {torch.float32: "f32", torch.bfloat16: "bf16", torch.float16: "f16"}[storage])
+    assert np.array_equal(both[0], out[0].cpu().numpy(), equal_nan=True)
     return out[0].cpu().numpy(), ref[0] if isinstance(ref, tuple) else ref
 
 
@@ -270,3 +277,15 @@ def test_rows_longest_detector_and_the_first_past_it(fan, det, copied):
     back = gh.backward2d(fan, sino, rays, (H, W), vo, vs, do, ds, **kw)
     ref = (orc.fan_backward if fan else orc.parallel_backward)(sino, rays, (H, W), vo, vs, do, ds, **kw)
     assert np.array_equal(back[0], ref[0] if isinstance(ref, tuple) else ref)
+
+
+@pytest.mark.parametrize("size, views", [(30, 28), (31, 27), (31, 17), (20, 16)])
+@pytest.mark.parametrize("fan", [False, True])
+def test_operators_on_both_sides_of_where_a_copy_pays(fan, size, views):
+    rng = np.random.default_rng(size)
+    got, ref = _run(fan, rng.normal(size=(size, size)).astype(np.float32), (1.0, 1.0), views, 40, 1.3 * size / 40, 1.0,
+                    1.6 * size)
+    assert np.array_equal(got, ref)
+    got, ref = _back(fan, rng.normal(size=(views, 40)).astype(np.float32), (size, size), (1.0, 1.0), 1.3 * size / 40,
+                     1.6 * size)
+    assert np.array_equal(got, ref)
