@@ -83,14 +83,20 @@ class _Plan(Capturable):
     def footprint(self) -> int:
         """Device bytes of one in-flight request: its input, the filtered copy, the GEMM
         filter's workspace (two float32 copies) if that filter is used, the detector cells
-        of the cone backprojection (four values per pixel) or the planar one's copy, and the
-        float32 output."""
+        of the cone backprojection (four values per pixel) or the planar one's copy where the
+        operator makes one, and the float32 output."""
         nin = int(np.prod(self.input_shape))
         nout = int(np.prod(self.output_shape))
         e = torch.tensor([], dtype=self.storage).element_size()
         ws = 8 if self.filter_impl == "gemm" else 0
-        cells = 4 * e if isinstance(self, ConeFDK) else e
-        return nin * (e + e + ws + cells) + nout * 4
+        if isinstance(self, ConeFDK):
+            copy = nin * 4 * e
+        else:
+            L, code, (n, det) = nat.lib(), _DT[self.storage], self.input_shape[-2:]
+            pays = L.pyronn_backprojection2d_copy_pays(isinstance(self, FanFBP), 1, n, det, code,
+                                                       *self.output_shape[-2:])
+            copy = L.pyronn_backprojection2d_workspace_size(1, n, det, code) if pays else 0
+        return nin * (e + e + ws) + copy + nout * 4
 
     def ramp_matrix(self) -> torch.Tensor:
         """The Toeplitz ramp matrix of the GEMM filter (built on first use)."""

@@ -23,6 +23,9 @@ import torch
 
 from . import geometry as geo
 from . import load as _load_ops
+from . import native as nat
+
+_DT = {torch.float32: nat.F32, torch.bfloat16: nat.BF16, torch.float16: nat.F16}
 
 
 def _cuda_device(device) -> torch.device:
@@ -30,6 +33,19 @@ def _cuda_device(device) -> torch.device:
     if d.type == "cuda" and d.index is None:
         d = torch.device("cuda", torch.cuda.current_device())
     return d
+
+
+def _planar_footprint(plan) -> int:
+    """Device bytes of one in-flight 2D projection: image, output, rays, and the pair copy of the
+    image where the operator makes one."""
+    g = plan.g
+    H, W = g.volume_shape
+    code = _DT[plan.storage]
+    L = nat.lib()
+    pairs = (L.pyronn_projection2d_workspace_size(1, H, W, code)
+             if L.pyronn_projection2d_copy_pays(1, H, W, code, g.n_views, g.detector_shape, plan.step_factor) else 0)
+    e = torch.tensor([], dtype=plan.storage).element_size()
+    return int(np.prod(plan.input_shape)) * e + pairs + int(np.prod(plan.output_shape)) * 4 + g.n_views * 8
 
 
 class Capturable:
@@ -119,11 +135,7 @@ class FanProjector(Capturable):
         self.output_shape = (1,) + tuple(g.projection_shape)
 
     def footprint(self) -> int:
-        e = torch.tensor([], dtype=self.storage).element_size()
-        H, W = self.g.volume_shape
-        pairs = (W + 4) * (H + 3) * 2 * e                    # the forward's pair copy
-        return (int(np.prod(self.input_shape)) * e + pairs + int(np.prod(self.output_shape)) * 4
-                + self.g.n_views * 8)
+        return _planar_footprint(self)
 
     def __call__(self, image: torch.Tensor) -> torch.Tensor:
         image = self._check_input(image)
@@ -153,11 +165,7 @@ class ParallelProjector(Capturable):
         self.output_shape = (1,) + tuple(g.projection_shape)
 
     def footprint(self) -> int:
-        e = torch.tensor([], dtype=self.storage).element_size()
-        H, W = self.g.volume_shape
-        pairs = (W + 4) * (H + 3) * 2 * e                    # the forward's pair copy
-        return (int(np.prod(self.input_shape)) * e + pairs + int(np.prod(self.output_shape)) * 4
-                + self.g.n_views * 8)
+        return _planar_footprint(self)
 
     def __call__(self, image: torch.Tensor) -> torch.Tensor:
         image = self._check_input(image)

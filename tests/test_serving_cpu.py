@@ -144,3 +144,35 @@ def test_grouping_respects_the_budget_and_group_max():
     Scheduler(ex2, slots=1, hbm_budget=100, group_max=2).run([Request(i, "g1", 0.0) for i in range(5)], clock=clk,
                                                              idle=clk.sleep)
     assert [len(g) for g in ex2.groups] == [2, 2]   # the last request runs alone through start()
+
+
+def _bare_plan(cls, g, storage, inp, out, **kw):
+    p = cls.__new__(cls)          # geometry and sizes only: a footprint asks for no device
+    p.g, p.storage, p.input_shape, p.output_shape = g, storage, inp, out
+    for k, v in kw.items():
+        setattr(p, k, v)
+    return p
+
+
+@pytest.mark.parametrize("side, views, pairs", [
+    (256, 180, 260 * 259 * 2 * 4),     # the pair copy: (W + 4)(H + 3) pairs
+    (4096, 100, 0),                    # too large for one
+    (16, 8, 0),                        # 16 samples a ray: sampled in place
+])
+def test_planar_projection_footprint_counts_the_copy_that_is_made(side, views, pairs):
+    import torch
+    from pyronn_layers import geometry as geo
+    from pyronn_layers.projectors import FanProjector, ParallelProjector
+    g = geo.Geometry2D((side, side), (1.0, 1.0), side, 1.5, views, sid=4.0 * side, sdd=5.0 * side, step_size=1.0)
+    for cls in (FanProjector, ParallelProjector):
+        p = _bare_plan(cls, g, torch.float32, (1, side, side), (1, views, side), step_factor=1.0)
+        assert p.footprint() == side * side * 4 + (pairs + 255) // 256 * 256 + views * side * 4 + views * 8
+
+
+@pytest.mark.parametrize("views, det, rows", [(360, 725, 360 * 729 * 2), (4, 725, 0), (40, 1 << 22, 0)])
+def test_planar_fbp_footprint_counts_the_copy_that_is_made(views, det, rows):
+    import torch
+    from pyronn_layers.fdk import FanFBP, ParallelFBP
+    for cls in (FanFBP, ParallelFBP):
+        p = _bare_plan(cls, None, torch.float16, (1, views, det), (1, 64, 64), filter_impl="fft")
+        assert p.footprint() == views * det * 4 + (rows + 255) // 256 * 256 + 64 * 64 * 4
