@@ -163,7 +163,7 @@ def test_planar_projection_footprint_counts_the_copy_that_is_made(side, views, p
     import torch
     from pyronn_layers import geometry as geo
     from pyronn_layers.projectors import FanProjector, ParallelProjector
-    g = geo.Geometry2D((side, side), (1.0, 1.0), side, 1.5, views, sid=4.0 * side, sdd=5.0 * side, step_size=1.0)
+    g = geo.Geometry2D((side, side), (1.0, 1.0), side, 1.5, views, 6.2832, sid=4.0 * side, sdd=5.0 * side, step_size=1.0)
     for cls in (FanProjector, ParallelProjector):
         p = _bare_plan(cls, g, torch.float32, (1, side, side), (1, views, side), step_factor=1.0)
         assert p.footprint() == side * side * 4 + (pairs + 255) // 256 * 256 + views * side * 4 + views * 8
