@@ -1199,8 +1199,9 @@ __global__ void __launch_bounds__(256, 5) cone_bp_items_kernel(BpBatch B) {
 // =====================================================================================
 // Host side
 // =====================================================================================
-// Elements the workspace holds for the cells: four per cell of the 16-bit layout, for f32 too
-// (whose x pairs fill about half of them).
+// Elements the workspace holds for the cells: four per cell of the 16-bit layout, for f32 too, whose x
+// pairs fill about half of them (1.09 of 2.18 GB at 512^3): callers keep the sizes that the query has
+// always given, and a smaller need is no reason to refuse theirs or to change what they read.
 static size_t cell_elems_dt(int, int D, int H, int W) { return cell_elems<bf16s>(D, H, W); }
 
 // Volumes the forward accepts: every side below 2^24 - 3, so that each cell coordinate and
@@ -1225,9 +1226,10 @@ template <typename TS> static bool fwd_byte_offsets(int D, int H, int W) {
   return W + 2 < (1 << 23) && 8 * plane < (1LL << 23) && 8 * (W + 2) * plane <= 0xB5000000LL;
 }
 // Cells the backprojection's workspace is sized for, four elements each; the two-element cells
-// fill about half of it.
+// fill about half of it (the size stays for the reason given at cell_elems_dt).
 static size_t det_cells(int n, int Hd, int Wd) { return (size_t)n * (Hd + 2) * (Wd + 2); }
-// Whether the backprojection may form its cell offsets in floats (sample_det).
+// Whether the backprojection may form its cell offsets in floats (det_fetch).  Beyond, integer offsets
+// cost little: 96 x 256 x 256 voxels, 24 views, detectors of 2896 x 2893 and 3072 x 3072, f32 1050 and 1215 us.
 static bool det_fidx(int Hd, int Wd) { return (long long)(Hd + 2) * det_cols(Wd) < (1LL << 23); }
 
 // A dispatch's grid size is a 32-bit count of work-items, so a 1-D grid of 256-lane blocks

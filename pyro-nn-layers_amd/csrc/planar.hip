@@ -925,10 +925,13 @@ static void launch_proj2d_g(dim3 grid, const void *volume, int dtype, int H, int
 
 // Rays per launch below which a ray gets 16 or 8 lanes instead of 4: a wave of a launch with few
 // rays issues an instruction every 8 cycles or so however independent they are, so a long ray's
-// time is its own instruction count; more lanes shorten it, at more additions per sample.
-// Measured with 4 / 8 / 16 lanes (us; parallel images, step 0.2): 2400 rays 12.7 / 9.6 / 8.4, 11400
-// 17.5 / 13.4 / 12.7, 12600 25.8 / 18.5 / 20.0, 38250 54.1 / 48.9 / 66.1, 65340 91.4 / 83.0 / 124.7,
-// 130680 137 / 142 / 211, 2.1 million 1388 / 1689 / 2912.
+// time is its own instruction count; more lanes shorten it, at more additions per sample.  The lines
+// lie where the launch fills the device, at 8 waves per SIMD (8192 waves: 65536 rays of 8 lanes; 12000
+// rays of 16 are 3 per SIMD, as their additions weigh more): waves beyond only add work.  Measured with 4 /
+// 8 / 16 lanes, us: parallel 256^2, step 0.2: 10890 rays 62 / 40 / 38, 21780 63 / 47 / 52, 50820 75 / 68 / 99,
+// 65340 85 / 78 / 121, 72600 87 / 86 / 130, 79860 85 / 95 / 140, 108900 115 / 122 / 180; rays a fifth as
+// long (step 1) 59895 21.2 / 21.0 / 30.7, 65340 23.1 / 22.8 / 32.6, 72600 23.4 / 24.1 / 34.9; fan 512^2, step
+// 0.5, 58000 64 / 58 / 92, 65250 63 / 66 / 100, bf16 66 / 62 and 69 / 72; 2.1 million rays 1388 / 1689 / 2912.
 constexpr long long kRowRays = 12000, kHalfRowRays = 65536;
 
 template <typename TS, bool FAN>
