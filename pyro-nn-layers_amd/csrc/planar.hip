@@ -716,9 +716,11 @@ back2d_kernel(const TS *__restrict__ sino, float *__restrict__ vol, const float 
 __host__ __device__ inline int row_len(int det) { return det + 4; }
 
 // 1 << lanes columns of 256 >> lanes rows per block and step (layout_lanes), four steps' loads in flight and
-// kRowsBlocks blocks at most, a device's worth: a copy of 189 MB (32 x 720 x 2048 f32) with one row per
-// block took about 150 us, now about 100.
-constexpr long long kRowsBlocks = 8192;
+// kRowsBlocks blocks at most, as many as the device holds.  A backprojection of 32 x 720 x 2048 f32 (189 MB
+// to copy) to 16 x 16 images: 238 us with one row per block, 316 / 242 / 181 / 184 / 188 with 512 / 1024 /
+// 2048 / 4096 / 8192 blocks; of one 180 x 363 image 24.7 with any.
+constexpr long long kRowsBlocks = 2048;
+
 template <typename TS>
 __global__ void __launch_bounds__(256)
 build_rows_kernel(const TS *__restrict__ sino, TS *__restrict__ rows, int det, long long nrows, int lanes) {
@@ -1184,8 +1186,7 @@ extern "C" size_t pyronn_backprojection2d_workspace_size(int batch, int n_views,
 // few and a view's chain is waited for, and 0.17 ps a pixel (fan 0.6) where they are many.  Measured in place
 // / through the copy, us a call: 256^2, 16 views 6.3 / 9.7 (fan 9.1 / 9.9), 32 views 10.3 / 9.6 (fan 16.3 /
 // 10.9); 1024^2, 8 views 9.7 / 10.7, 16 views 15.6 / 13.8; 8 of 512^2, 4 views 11.2 / 14.2, 12 views 22.0 / 19.8;
-// 32 sinograms of 720 x 2048 to 16 x 16 images f32 172 / 186, f16 220 / 128; 64 of 720 x 1024 to one pixel
-// 164 / 193; 4096 of 8 x 11 to 8 x 8 7.7 / 13.
+// 32 sinograms of 720 x 2048 to 16 x 16 images f32 172 / 181, f16 220 / 126; 4096 of 8 x 11 to 8 x 8 7.7 / 13.
 extern "C" int pyronn_backprojection2d_copy_pays(int fan, int batch, int n_views, int det, int sinogram_dtype, int H,
                                                  int W) {
   if (pyronn_backprojection2d_workspace_size(batch, n_views, det, sinogram_dtype) == 0 || H <= 0 || W <= 0) return 0;
