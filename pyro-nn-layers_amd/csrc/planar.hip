@@ -267,8 +267,9 @@ __device__ float march2d_group(const TS *__restrict__ img, int W, int H, float o
 // What bound the direct march (march2d above): about 100 VALU instructions per sample (the
 // neighbours' bounds tests, 64-bit addresses and selects of the shared-ray version, the
 // iteration cap) around loads whose latency nothing covered.  Here a sample takes 39, and a
-// wave's load 22 cycles of the texture-address unit (16 for one 128-byte line per quad):
-// that unit is 88% busy and VALU issue at 0.39 of its 0.44-0.5 per SIMD and cycle.  Parallel
+// wave's load 22 cycles of the texture-address unit (16 for one 128-byte line per quad): in a batch
+// that unit is 90% busy, the data-return unit 98% and VALU issue at 0.41 of its 0.5 per SIMD and cycle;
+// one image ends on its longest rays, with half its waves gone on average.  Parallel
 // 256^2 / 180 views x 363 / step 0.2: 32 images 4300 -> 1390 us, one 282 -> 83; fan 512^2 /
 // 360 x 725 / step 0.5: 535 -> 158; fan 301 x 277 f16, spacing 0.7, one image: 522 -> 124.
 // A second copy with x and y exchanged, for rays along y, was no faster (1496 us, 180 us):
@@ -701,12 +702,14 @@ back2d_kernel(const TS *__restrict__ sino, float *__restrict__ vol, const float 
 // holds s(-2) .. s(det + 1), zeros outside the detector, so a linear sample is one pair load
 // and no bounds test, the coordinate clamped into [-2, det].
 //
-// The fan kernel is bound by VALU issue.  back2d_kernel above forms about 130 instructions
-// per update: per-view terms of the line intersection that are the same for every pixel, two
+// The fan kernel takes its time in VALU instructions (a batch) and in waiting for each view's
+// chain of them (one 512^2 image, 4 waves per SIMD).  back2d_kernel above forms about 130 per
+// update: per-view terms of the line intersection that are the same for every pixel, two
 // IEEE divisions by one denominator, an IEEE square root and its reciprocal.  Here a block
 // forms the per-view terms once, in LDS (kBackViews views at a time; every lane reads them
 // back with two broadcast reads), both quotients share one correctly rounded reciprocal
-// (div_spacing's two corrections), and rcp_sqrt_fast serves the weight: about 68 per update.
+// (div_spacing's two corrections), and rcp_sqrt_fast serves the weight: 59 (detector spacing a
+// power of two) to 68 per update.
 // The parallel kernel's 15 leave it to the address path, one pair load per update.  With the
 // layout pass, 512^2 fan, 360 views x 725: 239 -> 135 us (8 images 1431 -> 872); 256^2 parallel, 180
 // views x 363: 49.5 -> 26 us (32 images 327 -> 178).  A test per view for the rare distances that
